@@ -45,50 +45,117 @@ __host__ __device__ inline float rcp_r(float x)
 #endif
 }
 
+// ------------------------------------------------------------ quotients
+// The binary64 kernels are bound by their arithmetic, and a division is the
+// dearest of it: the compiled sequence (scaling, reciprocal, Newton steps,
+// residual, fix-up) issues 11 operations, and divisions made up half to two
+// thirds of the binary64 operations of the chemistry, transport, collide and
+// moment kernels.  Most of their divisors are constants (molar masses) or shared
+// by many quotients (rho, T, a pivot), so a divisor carries its reciprocal
+// and a quotient takes three: the approximate quotient, its exact residual by
+// fused multiply-add and the correction (Markstein 1990).  The result is the
+// correctly rounded quotient (the error before the last rounding is below
+// 2^-51 units in the last place), so it is bit for bit that of `/`, for
+// divisors and quotients in the normal range; an infinite quotient or a zero
+// divisor gives NaN.  Host code divides.
+struct Divisor {
+    double b, y;  // the divisor and 1 / b to within 2^-52
+};
+// a / d.b by the residual correction
+__host__ __device__ inline double quotient_fma(double a, const Divisor& d)
+{
+    const double q = a * d.y;
+    const double r = __builtin_fma(-q, d.b, a);
+    return __builtin_fma(r, d.y, q);
+}
+// 1 / b: the hardware's approximate reciprocal and two Newton steps
+__host__ __device__ inline Divisor divisor(double b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+    y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+    return {b, y};
+#else
+    return {b, 1.0 / b};
+#endif
+}
+__host__ __device__ inline double quot(double a, const Divisor& d)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return quotient_fma(a, d);
+#else
+    return a / d.b;
+#endif
+}
+__host__ __device__ inline double quot(double a, double b) { return quot(a, divisor(b)); }
+// a / b of binary32 numbers through the binary64 reciprocal y of b: a
+// quotient of two 24-bit numbers is at least 2^-50 of itself away from the middle
+// of two binary32 numbers, so rounding a y (2^-52 off) gives the rounded quotient
+__host__ __device__ inline float quotf(float a, float b, double y)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (float)((double)a * y);
+#else
+    return a / b;
+#endif
+}
+// quotients by constants
+__host__ __device__ inline double third(double x) { return quot(x, Divisor{3.0, 1.0 / 3.0}); }
+__host__ __device__ inline double fifth(double x) { return quot(x, Divisor{5.0, 1.0 / 5.0}); }
+__host__ __device__ inline double over_w(double x, int k) { return quot(x, Divisor{W[k], INV_W_TABLE.v[k]}); }
+
 // ---------------------------------------------------------------- units
 // Units_Conv after set_m_kg_s(dx, dt): m, kg, s, K stored as float; every
 // conversion rounds its argument to float and computes in float, or in
 // double where the reference's double cb()/sq() enters, then returns float.
+// The y_ members are the reciprocals of the conversions' divisors for device
+// code (make_units sets them).
 struct Units {
     float m, kg, s, K;
+    double y_K = 0, y_mm = 0, y_ss = 0, y_m = 0, y_kg = 0, y_kgm = 0;  // binary32 divisors K, m m, s s, m, kg, kg m
+    double y_m3 = 0, y_m2 = 0, y_mss = 0;                              // binary64 divisors m^3, m^2, m s^2
 
-    __host__ __device__ float temp(double x) const { return (float)x / K; }
+    __host__ __device__ float temp(double x) const { return quotf((float)x, K, y_K); }
     __host__ __device__ float si_temp(double x) const { return (float)x * K; }
-    __host__ __device__ float energy_mass(double x) const { return (float)x * (s * s) / (m * m); }
-    __host__ __device__ float si_energy_mass(double x) const { return (float)x * (m * m) / (s * s); }
-    __host__ __device__ float u(double x) const { return (float)x * s / m; }  // velocity
+    __host__ __device__ float energy_mass(double x) const { return quotf((float)x * (s * s), m * m, y_mm); }
+    __host__ __device__ float si_energy_mass(double x) const { return quotf((float)x * (m * m), s * s, y_ss); }
+    __host__ __device__ float u(double x) const { return quotf((float)x * s, m, y_m); }  // velocity
     __host__ __device__ float rho(double x) const
     {
         const double md = m;
-        return (float)((double)(float)x * (md * md * md) / (double)kg);
+        return (float)quot((double)(float)x * (md * md * md), Divisor{(double)kg, y_kg});
     }
     __host__ __device__ float si_rho(double x) const
     {
         const double md = m;
-        return (float)((double)((float)x * kg) / (md * md * md));
+        return (float)quot((double)((float)x * kg), Divisor{md * md * md, y_m3});
     }
     __host__ __device__ float rho_dot(double x) const
     {
         const double md = m;
-        return (float)((double)(float)x * (md * md * md) * (double)s / (double)kg);
+        return (float)quot((double)(float)x * (md * md * md) * (double)s, Divisor{(double)kg, y_kg});
     }
     __host__ __device__ float nu(double x) const
     {
         const double md = m;
-        return (float)((double)((float)x * s) / (md * md));
+        return (float)quot((double)((float)x * s), Divisor{md * md, y_m2});
     }
-    __host__ __device__ float mu(double x) const { return (float)x * s * m / kg; }
-    __host__ __device__ float thermal_conductivity(double x) const { return (float)x * s * s * s * K / (kg * m); }
-    __host__ __device__ float cp(double x) const { return (float)x * s * s * K / (m * m); }
+    __host__ __device__ float mu(double x) const { return quotf((float)x * s * m, kg, y_kg); }
+    __host__ __device__ float thermal_conductivity(double x) const
+    {
+        return quotf((float)x * s * s * s * K, kg * m, y_kgm);
+    }
+    __host__ __device__ float cp(double x) const { return quotf((float)x * s * s * K, m * m, y_mm); }
     __host__ __device__ float p(double x) const
     {
         const double sd = s;
-        return (float)((double)(float)x * ((double)m * (sd * sd)) / (double)kg);
+        return (float)quot((double)(float)x * ((double)m * (sd * sd)), Divisor{(double)kg, y_kg});
     }
     __host__ __device__ float si_p(double x) const
     {
         const double sd = s;
-        return (float)((double)((float)x * kg) / ((double)m * (sd * sd)));
+        return (float)quot((double)((float)x * kg), Divisor{(double)m * (sd * sd), y_mss});
     }
 };
 
@@ -101,28 +168,91 @@ inline Units make_units(double dx, double dt)
     u.kg = (float)(1.0 / 1.0 * (md * md * md));
     u.s = (float)((double)(float)dt / 1.0);
     u.K = 12000.0f;
+    const float mm = u.m * u.m, ss = u.s * u.s, kgm = u.kg * u.m;
+    const double sd = u.s;
+    u.y_K = 1.0 / (double)u.K;
+    u.y_mm = 1.0 / (double)mm;
+    u.y_ss = 1.0 / (double)ss;
+    u.y_m = 1.0 / (double)u.m;
+    u.y_kg = 1.0 / (double)u.kg;
+    u.y_kgm = 1.0 / (double)kgm;
+    u.y_m3 = 1.0 / (md * md * md);
+    u.y_m2 = 1.0 / (md * md);
+    u.y_mss = 1.0 / ((double)u.m * (sd * sd));
     return u;
 }
 
 // --------------------------------------------------------------- thermo
-__host__ __device__ inline const double* nasa(int k, double T) { return T < T_MID[k] ? NASA_LO[k] : NASA_HI[k]; }
+// Rows of the coefficients a0..a6 and a2 / 3.
+struct NasaRows {
+    double v[NS][8];
+};
+constexpr NasaRows nasa_rows(const double (&t)[NS][7])
+{
+    NasaRows r{};
+    for (int k = 0; k < NS; ++k) {
+        for (int i = 0; i < 7; ++i) r.v[k][i] = t[k][i];
+        r.v[k][7] = t[k][2] / 3;
+    }
+    return r;
+}
+constexpr NasaRows ROWS_LO = nasa_rows(NASA_LO), ROWS_HI = nasa_rows(NASA_HI);
+__host__ __device__ inline const double* nasa(int k, double T) { return T < T_MID[k] ? ROWS_LO.v[k] : ROWS_HI.v[k]; }
 
+// Which side of T_MID the temperature lies on, as a branch.  Chosen by address,
+// a species' row is eight vector loads and as many register pairs per lane;
+// on either side of a branch the rows are constants in scalar registers, and
+// a wavefront runs both sides only when its lanes straddle T_MID.  Mechanisms
+// whose species differ in T_MID keep the choice by address.
+enum : int { SIDE_LO = 0, SIDE_HI = 1, SIDE_MIXED = 2 };
+template <int S>
+struct Side {
+    static constexpr int side = S;
+};
+constexpr bool one_t_mid()
+{
+    for (int k = 1; k < NS; ++k)
+        if (T_MID[k] != T_MID[0]) return false;
+    return true;
+}
+template <int S>
+__host__ __device__ inline const double* nasa_row(int k, double T)
+{
+    if constexpr (S == SIDE_LO) return ROWS_LO.v[k];
+    if constexpr (S == SIDE_HI) return ROWS_HI.v[k];
+    return nasa(k, T);
+}
+template <typename Body>
+__host__ __device__ inline void by_side(double T, Body body)
+{
+    if constexpr (one_t_mid()) {
+        if (T < T_MID[0]) body(Side<SIDE_LO>{});
+        else body(Side<SIDE_HI>{});
+    } else {
+        body(Side<SIDE_MIXED>{});
+    }
+}
+
+template <int S = SIDE_MIXED>
 __host__ __device__ inline double cp_R(int k, double T)
 {
-    const double* a = nasa(k, T);
+    const double* a = nasa_row<S>(k, T);
     return a[0] + T * (a[1] + T * (a[2] + T * (a[3] + T * a[4])));
 }
 
+template <int S = SIDE_MIXED>
 __host__ __device__ inline double h_RT(int k, double T)
 {
-    const double* a = nasa(k, T);
-    return a[0] + T * (a[1] / 2 + T * (a[2] / 3 + T * (a[3] / 4 + T * a[4] / 5))) + a[5] / T;
+    const double* a = nasa_row<S>(k, T);
+    const double t4 = fifth(T * a[4]);
+    return a[0] + T * (a[1] / 2 + T * (a[7] + T * (a[3] / 4 + t4))) + quot(a[5], T);
 }
 
+template <int S = SIDE_MIXED>
 __host__ __device__ inline double s_R(int k, double T, double lnT)
 {
-    const double* a = nasa(k, T);
-    return a[0] * lnT + T * (a[1] + T * (a[2] / 2 + T * (a[3] / 3 + T * a[4] / 4))) + a[6];
+    const double* a = nasa_row<S>(k, T);
+    return a[0] * lnT + T * (a[1] + T * (a[2] / 2 + T * (third(a[3]) + T * a[4] / 4))) + a[6];
 }
 
 // Cantera's setMassFractions: negatives clipped, then normalised.
@@ -134,7 +264,7 @@ __host__ __device__ inline void normalize(double Y[NS])
         Y[k] = Y[k] > 0.0 ? Y[k] : 0.0;
         s += Y[k];
     }
-    const double inv = 1.0 / s;
+    const double inv = quot(1.0, s);
 #pragma unroll
     for (int k = 0; k < NS; ++k) Y[k] *= inv;
 }
@@ -147,8 +277,8 @@ __host__ __device__ inline double mean_W(const double Y[NS])
 {
     double s = 0;
 #pragma unroll
-    for (int k = 0; k < NS; ++k) s += FAST ? Y[k] * inv_w(k) : Y[k] / W[k];
-    return 1.0 / s;
+    for (int k = 0; k < NS; ++k) s += FAST ? Y[k] * inv_w(k) : over_w(Y[k], k);
+    return quot(1.0, s);
 }
 
 template <bool FAST = false>
@@ -157,16 +287,17 @@ __host__ __device__ inline void X_from_Y(const double Y[NS], double X[NS])
     double s = 0;
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
-        X[k] = FAST ? Y[k] * inv_w(k) : Y[k] / W[k];
+        X[k] = FAST ? Y[k] * inv_w(k) : over_w(Y[k], k);
         s += X[k];
     }
     if constexpr (FAST) {
-        const double is = 1.0 / s;
+        const double is = quot(1.0, s);
 #pragma unroll
         for (int k = 0; k < NS; ++k) X[k] *= is;
     } else {
+        const Divisor ds = divisor(s);
 #pragma unroll
-        for (int k = 0; k < NS; ++k) X[k] /= s;
+        for (int k = 0; k < NS; ++k) X[k] = quot(X[k], ds);
     }
 }
 
@@ -178,32 +309,40 @@ __host__ __device__ inline void Y_from_X(const double X[NS], double Y[NS])
         Y[k] = (X[k] > 0.0 ? X[k] : 0.0) * W[k];
         s += Y[k];
     }
+    const Divisor ds = divisor(s);
 #pragma unroll
-    for (int k = 0; k < NS; ++k) Y[k] /= s;
+    for (int k = 0; k < NS; ++k) Y[k] = quot(Y[k], ds);
 }
 
 template <bool FAST = false>
 __host__ __device__ inline double cp_mass(double T, const double Y[NS])
 {
     double s = 0;
+    by_side(T, [&](auto sd) {
 #pragma unroll
-    for (int k = 0; k < NS; ++k) s += FAST ? Y[k] * cp_R(k, T) * inv_w(k) : Y[k] * cp_R(k, T) / W[k];
+        for (int k = 0; k < NS; ++k)
+            s += FAST ? Y[k] * cp_R<sd.side>(k, T) * inv_w(k) : over_w(Y[k] * cp_R<sd.side>(k, T), k);
+    });
     return s * R_UNIV;
 }
 
 // h / RT with the reciprocal temperature given (one division per state
 // instead of one per species)
+template <int S = SIDE_MIXED>
 __host__ __device__ inline double h_RT_inv(int k, double T, double invT)
 {
-    const double* a = nasa(k, T);
-    return a[0] + T * (a[1] / 2 + T * (a[2] / 3 + T * (a[3] / 4 + T * a[4] / 5))) + a[5] * invT;
+    const double* a = nasa_row<S>(k, T);
+    const double t4 = fifth(T * a[4]);
+    return a[0] + T * (a[1] / 2 + T * (a[7] + T * (a[3] / 4 + t4))) + a[5] * invT;
 }
 
 __host__ __device__ inline double u_mass(double T, const double Y[NS])
 {
     double s = 0;
+    by_side(T, [&](auto sd) {
 #pragma unroll
-    for (int k = 0; k < NS; ++k) s += Y[k] * (h_RT(k, T) - 1.0) / W[k];
+        for (int k = 0; k < NS; ++k) s += over_w(Y[k] * (h_RT<sd.side>(k, T) - 1.0), k);
+    });
     return s * R_UNIV * T;
 }
 
@@ -220,28 +359,34 @@ __host__ __device__ inline double T_from_UV(double u_target, const double Y[NS],
 #pragma unroll
         for (int k = 0; k < NS; ++k) yw[k] = Y[k] * inv_w(k);
         for (int it = 0; it < 60; ++it) {
-            const double invT = 1.0 / T;
+            const double invT = quot(1.0, T);
             double u = 0, cv = 0;
+            by_side(T, [&](auto sd) {
 #pragma unroll
-            for (int k = 0; k < NS; ++k) {
-                u += yw[k] * (h_RT_inv(k, T, invT) - 1.0);
-                cv += yw[k] * (cp_R(k, T) - 1.0);
-            }
-            const double dT = -(u * R_UNIV * T - u_target) / (cv * R_UNIV);
+                for (int k = 0; k < NS; ++k) {
+                    u += yw[k] * (h_RT_inv<sd.side>(k, T, invT) - 1.0);
+                    cv += yw[k] * (cp_R<sd.side>(k, T) - 1.0);
+                }
+            });
+            const double dT = quot(-(u * R_UNIV * T - u_target), cv * R_UNIV);
             T += dT;
             if (fabs(dT) <= 1e-15 * fabs(T)) break;
         }
         return T;
     }
+    double yw[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) yw[k] = over_w(Y[k], k);
     for (int it = 0; it < 60; ++it) {
         double u = 0, cv = 0;
+        by_side(T, [&](auto sd) {
 #pragma unroll
-        for (int k = 0; k < NS; ++k) {
-            const double yw = Y[k] / W[k];
-            u += yw * (h_RT(k, T) - 1.0);
-            cv += yw * (cp_R(k, T) - 1.0);
-        }
-        const double dT = -(u * R_UNIV * T - u_target) / (cv * R_UNIV);
+            for (int k = 0; k < NS; ++k) {
+                u += yw[k] * (h_RT<sd.side>(k, T) - 1.0);
+                cv += yw[k] * (cp_R<sd.side>(k, T) - 1.0);
+            }
+        });
+        const double dT = quot(-(u * R_UNIV * T - u_target), cv * R_UNIV);
         T += dT;
         if (fabs(dT) <= 1e-15 * fabs(T)) break;
     }
@@ -257,7 +402,7 @@ __host__ __device__ inline double pressure(double T, double rho, const double Y[
         for (int k = 0; k < NS; ++k) s += Y[k] * inv_w(k);
         return rho * R_UNIV * T * s;
     }
-    return rho * R_UNIV * T / mean_W(Y);
+    return quot(rho * R_UNIV * T, mean_W(Y));
 }
 
 // ------------------------------------------------------------ kinetics
@@ -303,14 +448,17 @@ constexpr bool any_plog()
 __host__ __device__ inline void net_production(double T, double rho, const double Y[NS], double wdot[NS])
 {
     double C[NS], gRT[NS];
-    const double lnT = log(T), invT = 1.0 / T;
+    const double lnT = log(T), invT = quot(1.0, T);
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
-        C[k] = rho * Y[k] / W[k];
-        gRT[k] = h_RT(k, T) - s_R(k, T, lnT);
+        C[k] = over_w(rho * Y[k], k);
         wdot[k] = 0.0;
     }
-    const double ln_pref_RT = log(P_REF / (R_UNIV * T));
+    by_side(T, [&](auto sd) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) gRT[k] = h_RT<sd.side>(k, T) - s_R<sd.side>(k, T, lnT);
+    });
+    const double ln_pref_RT = log(quot(P_REF, R_UNIV * T));
     // ln p of the PLOG rates, p = R T sum_k C_k
     double lnP = 0.0;
     if constexpr (any_plog()) {
@@ -321,34 +469,41 @@ __host__ __device__ inline void net_production(double T, double rho, const doubl
     }
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-        double kf = KIND[r] == 3 ? plog_rate(r, lnT, invT, lnP) : ARR_A[r] * exp(ARR_B[r] * lnT - ARR_EA_R[r] * invT);
+        // (a rate with b = 0 and Ea = 0 is A: exp(0) = 1 is not evaluated)
+        double kf = KIND[r] == 3                                ? plog_rate(r, lnT, invT, lnP)
+                    : ARR_B[r] == 0.0 && ARR_EA_R[r] == 0.0 ? ARR_A[r]
+                                                              : ARR_A[r] * exp(ARR_B[r] * lnT - ARR_EA_R[r] * invT);
         if (KIND[r] == 1 || KIND[r] == 2) {
             double M = 0;
 #pragma unroll
-            for (int k = 0; k < NS; ++k) M += EFF[r][k] * C[k];
+            for (int k = 0; k < NS; ++k)
+                if (EFF[r][k] != 0.0) M += EFF[r][k] * C[k];
             if (KIND[r] == 1) {
                 kf *= M;
             } else {
                 const double k0 = LOW_A[r] * exp(LOW_B[r] * lnT - LOW_EA_R[r] * invT);
-                const double Pr = k0 * M / kf;
+                const double Pr = quot(k0 * M, kf);
                 if (TROE_ON[r]) {
-                    double Fc = (1.0 - TROE[r][0]) * exp(-T / TROE[r][1]) + TROE[r][0] * exp(-T / TROE[r][2]);
+                    double Fc = (1.0 - TROE[r][0]) * exp(quot(-T, Divisor{TROE[r][1], 1.0 / TROE[r][1]})) +
+                                TROE[r][0] * exp(quot(-T, Divisor{TROE[r][2], 1.0 / TROE[r][2]}));
                     if (TROE_HAS_T2[r]) Fc += exp(-TROE[r][3] * invT);
                     const double lFc = log10(Fc);
                     const double lPr = log10(Pr > 1e-300 ? Pr : 1e-300);
                     const double cc = -0.4 - 0.67 * lFc;
                     const double nn = 0.75 - 1.27 * lFc;
-                    const double f1 = (lPr + cc) / (nn - 0.14 * (lPr + cc));
-                    kf = kf * Pr / (1.0 + Pr) * exp10(lFc / (1.0 + f1 * f1));
+                    const double f1 = quot(lPr + cc, nn - 0.14 * (lPr + cc));
+                    kf = quot(kf * Pr, 1.0 + Pr) * exp10(quot(lFc, 1.0 + f1 * f1));
                 } else {  // Lindemann: broadening factor 1
-                    kf = kf * Pr / (1.0 + Pr);
+                    kf = quot(kf * Pr, 1.0 + Pr);
                 }
             }
         }
         double dG = 0, dn = 0, cf = 1, cr = 1;
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
-            dG += (NU_R[r][k] - NU_F[r][k]) * gRT[k];
+            // species the reaction leaves alone add nothing (the table's zeros
+            // do not fold by themselves: 0 x is not 0 for every x)
+            if (NU_R[r][k] - NU_F[r][k] != 0.0) dG += (NU_R[r][k] - NU_F[r][k]) * gRT[k];
             dn += NU_R[r][k] - NU_F[r][k];
             cf *= conc_power(C[k], ORD_F[r][k]);
             cr *= conc_power(C[k], NU_R[r][k]);
@@ -373,7 +528,7 @@ __host__ __device__ inline double species_conductivity(int k, double lnT) { retu
 // D_ab [m^2/s] at (T, p).
 __host__ __device__ inline double binary_diff(int a, int b, double lnT, double p)
 {
-    return exp(poly4(DIFF_FIT[a][b], lnT)) / p;
+    return quot(exp(poly4(DIFF_FIT[a][b], lnT)), p);
 }
 
 // The same fits evaluated in arithmetic type R (double reproduces the
@@ -392,7 +547,14 @@ template <typename R>
 __host__ __device__ inline R binary_diff_r(int a, int b, R lnT, R p)
 {
     if constexpr (sizeof(R) == 4) return exp(poly4r<R>(DIFF_FIT[a][b], lnT)) * rcp_r(p);
-    return exp(poly4r<R>(DIFF_FIT[a][b], lnT)) / p;
+    return quot(exp(poly4r<R>(DIFF_FIT[a][b], lnT)), p);
+}
+
+// Divisor sqrt(8 (1 + W_a / W_b)) of the Wilke weights
+__host__ __device__ inline Divisor wilke_divisor(int a, int b)
+{
+    const double d = sqrt(8.0 * (1.0 + W[a] / W[b]));
+    return {d, 1.0 / d};
 }
 
 // Wilke weight Phi_ab with sqrt(mu_a / mu_b) given: (1 + sqrt(mu_a/mu_b)
@@ -446,19 +608,27 @@ __host__ __device__ inline R mix_viscosity_r(R lnT, const double X[NS])
         }
         return tot;
     }
-    R mu[NS];
+    double mu[NS];
+    Divisor dmu[NS];
 #pragma unroll
-    for (int k = 0; k < NS; ++k) mu[k] = species_viscosity_r<R>(k, lnT);
-    R tot = 0;
+    for (int k = 0; k < NS; ++k) {
+        mu[k] = species_viscosity(k, lnT);
+        dmu[k] = divisor(mu[k]);
+    }
+    double tot = 0;
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
-        R den = 0;
+        double den = 0;
 #pragma unroll
         for (int b = 0; b < NS; ++b) {
-            const R r = R(1) + sqrt(mu[a] / mu[b]) * (R)sqrt(sqrt(W[b] / W[a]));
-            den += (R)X[b] * (r * r / (R)sqrt(8.0 * (1.0 + W[a] / W[b])));
+            if (b == a) {  // Phi_aa = 1
+                den += X[a];
+                continue;
+            }
+            const double r = 1.0 + sqrt(quot(mu[a], dmu[b])) * sqrt(sqrt(W[b] / W[a]));
+            den += X[b] * quot(r * r, wilke_divisor(a, b));
         }
-        tot += (R)X[a] * mu[a] / den;
+        tot += quot(X[a] * mu[a], den);
     }
     return tot;
 }
@@ -474,10 +644,10 @@ __host__ __device__ inline R mix_conductivity_r(R lnT, const XT X[NS])
         if constexpr (sizeof(R) == 4)
             s2 += (R)X[k] * rcp_r(l);
         else
-            s2 += (R)X[k] / l;
+            s2 += quot((double)X[k], (double)l);
     }
     if constexpr (sizeof(R) == 4) return R(0.5) * (s1 + rcp_r(s2));
-    return R(0.5) * (s1 + R(1) / s2);
+    return R(0.5) * (s1 + R(quot(1.0, (double)s2)));
 }
 
 // Combination-averaged mixture conductivity 1/2 (sum X l + 1 / sum X / l).

@@ -148,10 +148,6 @@ struct lbm_ctx {
     unsigned* chem_list = nullptr;
     unsigned* chem_count = nullptr;
     double* tchem = nullptr;
-    uint16_t* sur_x = nullptr;  // in-step network inputs [sur_rows][16] BF16
-    float* sur_y = nullptr;     // outputs [sur_rows][16]
-    uint8_t* sur_flag = nullptr;
-    int64_t sur_rows = 0;
     float* cap_buf = nullptr;
     unsigned long long* cap_count = nullptr;
     long long cap_max = 0;
@@ -484,7 +480,7 @@ void release(lbm_ctx* c)
                     c->sf[1],     c->sp_block,  c->tms_cell,   c->tms_dir,   c->src,       c->sur_stats,
                     c->stats_part, c->sur_count, c->chem_list, c->chem_count, c->tchem,    c->cap_buf,
                     c->cap_count, c->bx,        c->bt,         c->bloss,     c->mref_dev,  c->sums_part, c->adam_c12, c->train_it,
-                    c->sur_x,     c->sur_y,     c->sur_flag,  c->tin_cell,  c->tin_dir,   c->sbc_cell,  c->tsp,        c->omix,       c->twall_cell, c->cjc_cell,
+                    c->tin_cell,  c->tin_dir,   c->sbc_cell,  c->tsp,        c->omix,       c->twall_cell, c->cjc_cell,
                     c->side_slot, c->side_cell, c->fside, c->aa_pending, c->low_cell, c->low_sp,
                     c->low_keep,  c->low_count, c->smooth_tmp, c->tms_rec};
     for (void* p : ptrs)
@@ -1536,8 +1532,7 @@ int lbm_collide_species(lbm_ctx* c)
             rc = DISPATCH(c, [&] {
                 const MultiView<P> v = make_mview<P>(c, 0, 1);
                 int r = launch(c, "mc_chemistry_surrogate", [&] {
-                    launch_mc_sur_chemistry<P>(v, c->net, c->sur_x, c->sur_y, c->sur_flag, c->sur_rows,
-                                               c->chem_list, c->chem_count, c->stream);
+                    launch_mc_sur_chemistry<P>(v, c->net, c->chem_list, c->chem_count, c->stream);
                 });
                 if (!r)
                     r = launch(c, "mc_chemistry_fallback",
@@ -1713,8 +1708,8 @@ int lbm_moments(lbm_ctx* c)
 
 namespace {
 
-// Collide_Species and Collide of one fused-mode reacting step with the
-// chemistry on a second stream.  The chemistry reads the fields and species
+// Collide_Species and Collide of one reacting step with the chemistry on a
+// second stream.  The chemistry reads the fields and species
 // planes of the last calculate_moment and writes only its own outputs
 // (sources, heat release, the fallback list, capture rows); the transport
 // pass and the mixture collide neither read nor write those, so the whole
@@ -1749,10 +1744,9 @@ int collide_overlapped(lbm_ctx* c)
         const MultiView<P> v = make_mview<P>(c, 0, 1);
         if (!c->sur_on)
             return launch_on(c, c->cstream, "mc_chemistry_plain",
-                             [&] { launch_mc<P>(McKernel::Chemistry, v, c->cstream); });
+                             [&] { launch_mc<P>(McKernel::ChemistryBeside, v, c->cstream); });
         int r = launch_on(c, c->cstream, "mc_chemistry_surrogate", [&] {
-            launch_mc_sur_chemistry<P>(v, c->net, c->sur_x, c->sur_y, c->sur_flag, c->sur_rows, c->chem_list,
-                                       c->chem_count, c->cstream);
+            launch_mc_sur_chemistry<P>(v, c->net, c->chem_list, c->chem_count, c->cstream);
         });
         if (!r)
             r = launch_on(c, c->cstream, "mc_chemistry_fallback",
@@ -1767,9 +1761,11 @@ int collide_overlapped(lbm_ctx* c)
     HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_cdone, 0));
     if (!rc && inplace(c)) {
         rc = aa_collide_species(c);
-    } else if (!rc) {
+    } else if (!rc && fused(c) && c->push_ready) {
         rc = run_mc(c, McKernel::CollideSpeciesPush, "mc_collide_species_push", 0, 1);
         if (!rc) c->pushed = true;
+    } else if (!rc) {
+        rc = run_mc(c, McKernel::CollideSpecies, "mc_collide_species", 0, 1);
     }
     ++c->step;
     return rc;
@@ -1782,10 +1778,8 @@ int lbm_step(lbm_ctx* c, int nsteps)
     if (!c) return LBM_E_ARG;
     for (int s = 0; s < nsteps; ++s) {
         int rc;
-        // the overlapped schedule covers the fused mode's pushed steps and the
-        // in-place mode, with chemistry
-        const bool ov = c->overlap && multi(c) && c->types_set && c->cfg.reaction &&
-                        ((fused(c) && c->push_ready) || inplace(c));
+        // every multicomponent step with chemistry takes the overlapped schedule
+        const bool ov = c->overlap && multi(c) && c->types_set && c->cfg.reaction;
         if (ov) {
             if ((rc = collide_overlapped(c))) return rc;
         } else if ((rc = lbm_collide_species(c)) || (rc = lbm_collide(c))) {
@@ -2245,16 +2239,10 @@ int lbm_surrogate_enable(lbm_ctx* c, int on, int audit_stride, double audit_tol)
     if (!c->norm_ready) return fail(c, LBM_E_STATE, "train the surrogate (or set its normalisation) first");
     const int64_t n = c->d.n;
     if (!c->chem_list) {
-        c->sur_rows = (n + 255) / 256 * 256;
         HIP_TRY(c, hipMalloc((void**)&c->chem_list, sizeof(unsigned) * n));
         HIP_TRY(c, hipMalloc((void**)&c->chem_count, sizeof(unsigned)));
         HIP_TRY(c, hipMalloc((void**)&c->tchem, sizeof(double) * n));
-        HIP_TRY(c, hipMalloc((void**)&c->sur_x, sizeof(uint16_t) * 16 * c->sur_rows));
-        HIP_TRY(c, hipMalloc((void**)&c->sur_y, sizeof(float) * 16 * c->sur_rows));
-        HIP_TRY(c, hipMalloc((void**)&c->sur_flag, n));
-        HIP_TRY(c, hipMemsetAsync(c->sur_x, 0, sizeof(uint16_t) * 16 * c->sur_rows, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-        c->bytes += (sizeof(unsigned) + sizeof(double) + 1) * n + (2 + 4) * 16 * c->sur_rows;
+        c->bytes += (sizeof(unsigned) + sizeof(double)) * n;
     }
     c->audit_stride = audit_stride;
     c->audit_tol = (float)audit_tol;

@@ -83,7 +83,9 @@ constexpr unsigned CHEM_AUDIT = 0x80000000u;
 // species sets in fo from the streamed f.
 // SpeciesTransport runs first in Collide_Species (per cell: omega_a and the
 // Maxwell-Stefan friction), then CollideSpecies or CollideSpeciesPush.
-enum class McKernel { Init, Chemistry, SpeciesTransport, CollideSpecies, Collide, Stream, Moments, CollideSpeciesPush,
+// ChemistryBeside is Chemistry launched to share the CUs with the kernels of
+// another stream.
+enum class McKernel { Init, Chemistry, ChemistryBeside, SpeciesTransport, CollideSpecies, Collide, Stream, Moments, CollideSpeciesPush,
                       StreamEnergy, SideFill, Unstream };
 
 template <typename P>
@@ -134,14 +136,14 @@ void launch_mc_tms_in(const MultiView<P>& v, const int* cells, const int* dirs, 
 template <typename P>
 void launch_mc_tms_wall(const MultiView<P>& v, const int* cells, int count, hipStream_t s);
 
-// Surrogate chemistry of every fluid cell: features (BF16 [rows][16] in X,
-// envelope flags), network (BF16 MFMA, FP32 outputs [rows][16] in Y; rows >=
-// n, a multiple of 256, rows past n zero), decoded sources into v.src /
-// v.hrr / v.tchem; cells outside the training envelope and the audited
-// chunks are appended to `list` (count in *count, zeroed first on the stream).
+// Surrogate chemistry of every fluid cell in one pass: normalised BF16 features
+// and envelope test, network (BF16 MFMA, FP32 outputs), decoded sources into
+// v.src / v.hrr / v.tchem; cells outside the training envelope and the
+// audited chunks are appended to `list` (count in *count, zeroed first on the
+// stream).
 template <typename P>
-void launch_mc_sur_chemistry(const MultiView<P>& v, const sur::Mlp& net, uint16_t* X, float* Y, uint8_t* flag,
-                             int64_t rows, unsigned* list, unsigned* count, hipStream_t s);
+void launch_mc_sur_chemistry(const MultiView<P>& v, const sur::Mlp& net, unsigned* list, unsigned* count,
+                             hipStream_t s);
 // Plain chemistry of the listed cells: fallbacks are overwritten, audits are
 // compared with the network's result and overwritten above the tolerance.
 template <typename P>

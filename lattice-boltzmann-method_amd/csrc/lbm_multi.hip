@@ -293,21 +293,22 @@ __device__ inline void chem_state(const MultiView<P>& v, int c, bool with_energy
 {
     const int64_t n = v.d.n;
     s.rho = v.fld[LBM_FIELD_RHO][c];
+    const Divisor drho = divisor(s.rho);
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
         s.ra[a] = v.rhoa[a * n + c];
-        s.Y0[a] = s.ra[a] / s.rho;
+        s.Y0[a] = quot(s.ra[a], drho);
     }
     normalize(s.Y0);
     s.Tsi = v.u.si_temp(v.fld[LBM_FIELD_T][c]);
     s.rho_si = v.u.si_rho(s.rho);
     s.usi = 0.0;
     if (with_energy) {
-        double Uint = v.fld[LBM_FIELD_RHOE][c] / s.rho;
+        double Uint = quot(v.fld[LBM_FIELD_RHOE][c], drho);
         for (int a = 0; a < NS; ++a) {
             const double ux = v.ua[(0 * NS + a) * n + c], uy = v.ua[(1 * NS + a) * n + c],
                          uz = v.ua[(2 * NS + a) * n + c];
-            Uint = Uint - 0.5 * s.ra[a] / s.rho * (ux * ux + uy * uy + uz * uz);
+            Uint = Uint - quot(0.5 * s.ra[a], drho) * (ux * ux + uy * uy + uz * uz);
         }
         s.usi = v.u.si_energy_mass(Uint);
     }
@@ -321,6 +322,7 @@ template <typename P>
 __device__ inline void plain_chemistry(const MultiView<P>& v, const ChemState& s, double src[NS], double* Tout)
 {
     double Tcur = s.Tsi, Ycur[NS];
+    const Divisor drho = divisor(s.rho);
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
         Ycur[a] = s.Y0[a];
@@ -332,7 +334,7 @@ __device__ inline void plain_chemistry(const MultiView<P>& v, const ChemState& s
 #pragma unroll
         for (int a = 0; a < NS; ++a) {
             src[a] += 1.0 / 2.0 * (double)v.u.rho_dot(wdot[a] * W[a]);
-            Ycur[a] = (s.ra[a] + src[a]) / s.rho;
+            Ycur[a] = quot(s.ra[a] + src[a], drho);
         }
         normalize(Ycur);
         Tcur = T_from_UV(s.usi, Ycur, Tcur);
@@ -345,8 +347,11 @@ template <typename P>
 __device__ inline double heat_release(const MultiView<P>& v, const double src[NS], double T)
 {
     double hrr = 0;
+    by_side(T, [&](auto sd) {
 #pragma unroll
-    for (int a = 0; a < NS; ++a) hrr += -1.0 * (double)v.u.energy_mass(h_RT(a, T) * R_UNIV * T / W[a]) * src[a];
+        for (int a = 0; a < NS; ++a)
+            hrr += -1.0 * (double)v.u.energy_mass(over_w(h_RT<sd.side>(a, T) * R_UNIV * T, a)) * src[a];
+    });
     return hrr;
 }
 
@@ -384,10 +389,19 @@ __device__ inline void capture_row(const MultiView<P>& v, const ChemState& s, co
     for (int q = 16 + sur::NOUT; q < 32; ++q) row[q] = 0.f;
 }
 
+// waves per SIMD the plain chemistry is built for (a large mechanism's
+// per-cell arrays would spill)
+constexpr int CHEM_WAVES = NS <= 16 ? 3 : 1;
+
 // Plain chemistry of every fluid cell; optionally samples (state, result)
-// rows for the surrogate's training set.
+// rows for the surrogate's training set.  Bound by its binary64 arithmetic (46
+// exponentials a sub-step).  With quotients by residual correction, the
+// thermo rows as constants of a branch (by_side) and literals left where
+// they are used (the build's -disable-machine-licm) it fits three waves per
+// SIMD (168 VGPRs, 28 B of scratch; 405 and one wave before): 368 -> 149 us on
+// 128x96x48 cells in FP64, 575 -> 222 us on 131x97x75 in FP32.
 template <typename P>
-__global__ __launch_bounds__(BLOCK) void k_mc_chemistry(MultiView<P> v)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CHEM_WAVES, 8))) void k_mc_chemistry(MultiView<P> v)
 {
     const int c = blockIdx.x * BLOCK + threadIdx.x;
     if (c >= v.d.n || v.type[c] != TYPE_F) return;
@@ -399,107 +413,168 @@ __global__ __launch_bounds__(BLOCK) void k_mc_chemistry(MultiView<P> v)
     if (v.cap_buf && mix_hash(c, v.step) % (unsigned)v.cap_stride == 0) capture_row(v, s, src, Tcur);
 }
 
-// Surrogate chemistry in three passes, so that the FP64 feature and decode
-// work runs at full occupancy and the network pass is pure matrix-core work:
-//   k_mc_sur_features: normalised BF16 features [n][16] and envelope flags;
-//   sur::mlp_infer_bf16: the network, outputs [n][16] FP32;
-//   k_mc_sur_decode: sources, HRR and final temperature; cells outside the
-//   envelope and audited 32-cell chunks go to the plain integrator's list.
-template <typename P>
-__global__ __launch_bounds__(BLOCK) void k_mc_sur_features(MultiView<P> v, uint16_t* X, uint8_t* flag)
+// Surrogate chemistry of every fluid cell in one pass: features, network,
+// decoded sources; cells outside the envelope and audited 32-cell chunks go to
+// the plain integrator's list.  A wavefront takes 64 cells: each lane forms its
+// cell's normalised BF16 features (binary64 state), the wavefront evaluates two
+// 32-row halves of the network from LDS, and each lane decodes its cell's
+// outputs, with rho and T still in registers.  As three kernels the inputs
+// (32 B a cell) and outputs (64 B) went through memory and each cell's state
+// was read and normalised twice: 950 us on 256x128x128 cells with the list's
+// kernel aside, 760 us fused with as many wavefronts.
+// One block per CU holds the weights (72 KiB) once and 4 KiB a wavefront for the
+// rows.  Eight wavefronts (two per SIMD) leave almost half of the registers
+// to the transport pass and the mixture collide that run beside it: a step
+// of 256x128x128 cells takes 6.70 ms, with sixteen 6.82, with eight of 64 rows
+// at a time (242 VGPRs, the whole file) 6.85.
+constexpr int SUR_WAVES = 8;
+
+// A value that is the same in every lane, in scalar registers.
+__device__ inline double uniform(double x)
 {
-    using namespace sur;
-    const int c = blockIdx.x * BLOCK + threadIdx.x;
-    if (c >= v.d.n) return;
-    const float* st = v.sur_stats;
-    float raw[NIN] = {};
-    const bool mine = v.type[c] == TYPE_F;
-    if (mine) {
-        ChemState s;
-        chem_state(v, c, false, s);
-        raw[0] = (float)s.Tsi;
-        raw[1] = (float)pressure(s.Tsi, s.rho_si, s.Y0);
-#pragma unroll
-        for (int a = 0; a < NS; ++a) raw[2 + a] = (float)s.Y0[a];
-        raw[NIN - 1] = v.u.s;
-    }
-    bool outside = false;
-    uint32_t packed[8];
-#pragma unroll
-    for (int q = 0; q < 16; q += 2) {
-        float x0 = 0.f, x1 = 0.f;
-        if (mine && q < NIN) {
-            outside |= raw[q] < st[SS_LO + q] || raw[q] > st[SS_HI + q];
-            x0 = (raw[q] - st[SS_FMEAN + q]) / st[SS_FSTD + q];
-        }
-        if (mine && q + 1 < NIN) {
-            outside |= raw[q + 1] < st[SS_LO + q + 1] || raw[q + 1] > st[SS_HI + q + 1];
-            x1 = (raw[q + 1] - st[SS_FMEAN + q + 1]) / st[SS_FSTD + q + 1];
-        }
-        packed[q / 2] = (uint32_t)f2bf(x0) | ((uint32_t)f2bf(x1) << 16);
-    }
-    uint4* dst = reinterpret_cast<uint4*>(X + (int64_t)c * 16);
-    dst[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-    dst[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
-    flag[c] = outside ? 1 : 0;
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 template <typename P>
-__global__ __launch_bounds__(BLOCK) void k_mc_sur_decode(MultiView<P> v, const float* Y, const uint8_t* flag,
-                                                         unsigned* list, unsigned* count)
+__global__ __launch_bounds__(SUR_WAVES * 64)
+void k_mc_surrogate(MultiView<P> v, sur::Mlp net, unsigned* list, unsigned* count)
 {
     using namespace sur;
+    __shared__ __align__(16) uint16_t Wf[FRAG_TOTAL];
+    __shared__ float bias[BIAS_TOTAL];
+    __shared__ __align__(16) float rows[SUR_WAVES][64 * 16];  // BF16 inputs, then FP32 outputs
     __shared__ unsigned blk_used, blk_fb;
+    if (threadIdx.x == 0) blk_used = blk_fb = 0u;
+    stage_net(net, Wf, bias);
+    __syncthreads();
     const int64_t n = v.d.n;
     const float* st = v.sur_stats;
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x == 0) blk_used = blk_fb = 0u;
-    __syncthreads();
-    const int c = blockIdx.x * BLOCK + threadIdx.x;
-    const bool mine = c < n && v.type[c] == TYPE_F;
-    bool audit = false, fallback = false;
-    if (mine) {
-        ChemState s;
-        chem_state(v, c, false, s);
-        const float4* pr4 = reinterpret_cast<const float4*>(Y + (int64_t)c * 16);
-        const float4 y0 = pr4[0], y1 = pr4[1], y2 = pr4[2];
-        static_assert(!sur::ENABLED || NOUT <= 12, "three float4 loads cover the real outputs");
-        const float pr[12] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w, y2.x, y2.y, y2.z, y2.w};
-        // the imbalance of the predicted sources is removed in proportion to each
-        // species' target scale (an inert species, scale 0, keeps its mean)
-        double src[NS], sum = 0, wsum = 0;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    float* const yout = rows[wave];
+    uint16_t* const xin = reinterpret_cast<uint16_t*>(yout);
+    unsigned n_used = 0, n_fb = 0;
+    // the record's quotients, once per wavefront and in scalar registers: 1 /
+    // scale of each feature, each species' share of the sources' imbalance
+    double y_std[NIN], share[NS], wsum = 0;
 #pragma unroll
-        for (int a = 0; a < NS; ++a) {
-            src[a] = s.rho * ((double)pr[1 + a] * st[SS_TSTD + 1 + a] + st[SS_TMEAN + 1 + a]);
-            sum += src[a];
-            wsum += st[SS_TSTD + 1 + a];
+    for (int q = 0; q < NIN; ++q) y_std[q] = uniform(1.0 / (double)st[SS_FSTD + q]);
+#pragma unroll
+    for (int a = 0; a < NS; ++a) wsum += st[SS_TSTD + 1 + a];
+#pragma unroll
+    for (int a = 0; a < NS; ++a) share[a] = uniform(st[SS_TSTD + 1 + a] / wsum);
+    const int64_t stride = (int64_t)gridDim.x * SUR_WAVES * 64;
+    // consecutive groups go to the blocks in turn, so that the last, partial round
+    // is spread over all of them
+    for (int64_t base = ((int64_t)wave * gridDim.x + blockIdx.x) * 64; base < n; base += stride) {
+        const int64_t c64 = base + lane;
+        const int c = (int)(c64 < n ? c64 : n - 1);
+        const bool mine = c64 < n && v.type[c] == TYPE_F;
+        if (!__ballot(mine)) continue;
+        double rho = 1.0, Tsi = 0.0;
+        bool outside = false;
+        {
+            float raw[NIN] = {};
+            if (mine) {
+                ChemState s;
+                chem_state(v, c, false, s);
+                rho = s.rho;
+                Tsi = s.Tsi;
+                raw[0] = (float)s.Tsi;
+                raw[1] = (float)pressure(s.Tsi, s.rho_si, s.Y0);
+#pragma unroll
+                for (int a = 0; a < NS; ++a) raw[2 + a] = (float)s.Y0[a];
+                raw[NIN - 1] = v.u.s;
+            }
+            uint32_t packed[8];
+#pragma unroll
+            for (int q = 0; q < 16; q += 2) {
+                float x0 = 0.f, x1 = 0.f;
+                if (q < NIN) {
+                    outside |= raw[q] < st[SS_LO + q] || raw[q] > st[SS_HI + q];
+                    x0 = quotf(raw[q] - st[SS_FMEAN + q], st[SS_FSTD + q], y_std[q]);
+                }
+                if (q + 1 < NIN) {
+                    outside |= raw[q + 1] < st[SS_LO + q + 1] || raw[q + 1] > st[SS_HI + q + 1];
+                    x1 = quotf(raw[q + 1] - st[SS_FMEAN + q + 1], st[SS_FSTD + q + 1], y_std[q + 1]);
+                }
+                packed[q / 2] = (uint32_t)f2bf(x0) | ((uint32_t)f2bf(x1) << 16);
+            }
+            uint4* dst = reinterpret_cast<uint4*>(xin + lane * 16);
+            dst[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+            dst[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
         }
+        // the rows pass between the lanes of this wavefront only: its LDS
+        // operations complete in order, the fences keep the compiler to it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        v4s x[4];
 #pragma unroll
-        for (int a = 0; a < NS; ++a) src[a] -= st[SS_TSTD + 1 + a] / wsum * sum;  // no net mass
-        const double Tcur = s.Tsi + ((double)pr[0] * st[SS_TSTD] + st[SS_TMEAN]);
-        const bool finite = isfinite(sum) && isfinite(Tcur) && Tcur > 0.0;
-        fallback = flag[c] != 0 || !finite;
-        if (!finite) {
-#pragma unroll
-            for (int a = 0; a < NS; ++a) src[a] = 0.0;
+        for (int bt = 0; bt < 4; ++bt) x[bt] = input_frag(xin, bt);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 1
+        for (int h = 0; h < 2; ++h) {
+            // keeps the weight fragments' LDS reads inside the loop (hoisted out
+            // of it they would need 576 registers)
+            asm volatile("" ::: "memory");
+            const v4s xh[2] = {h ? x[2] : x[0], h ? x[3] : x[1]};
+            v4f y[2];
+            mlp_rows32(Wf, bias, xh, y);
+            output_frag(yout, 2 * h, y[0]);
+            output_frag(yout, 2 * h + 1, y[1]);
         }
-        store_chem(v, c, src, finite ? Tcur : s.Tsi);
-        audit = !fallback && v.audit_stride > 0 && mix_hash((unsigned)(c >> 5), v.step) % (unsigned)v.audit_stride == 0;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        bool audit = false, fallback = false;
+        if (mine) {
+            const float4* pr4 = reinterpret_cast<const float4*>(yout + lane * 16);
+            const float4 y0 = pr4[0], y1 = pr4[1], y2 = pr4[2];
+            static_assert(!sur::ENABLED || NOUT <= 12, "three float4 loads cover the real outputs");
+            const float pr[12] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w, y2.x, y2.y, y2.z, y2.w};
+            // the imbalance of the predicted sources is removed in proportion to each
+            // species' target scale (an inert species, scale 0, keeps its mean)
+            double src[NS], sum = 0;
+#pragma unroll
+            for (int a = 0; a < NS; ++a) {
+                src[a] = rho * ((double)pr[1 + a] * st[SS_TSTD + 1 + a] + st[SS_TMEAN + 1 + a]);
+                sum += src[a];
+            }
+#pragma unroll
+            for (int a = 0; a < NS; ++a) src[a] -= share[a] * sum;  // no net mass
+            const double Tcur = Tsi + ((double)pr[0] * st[SS_TSTD] + st[SS_TMEAN]);
+            const bool finite = isfinite(sum) && isfinite(Tcur) && Tcur > 0.0;
+            fallback = outside || !finite;
+            if (!finite) {
+#pragma unroll
+                for (int a = 0; a < NS; ++a) src[a] = 0.0;
+            }
+            store_chem(v, c, src, finite ? Tcur : Tsi);
+            audit = !fallback && v.audit_stride > 0 &&
+                    mix_hash((unsigned)(c >> 5), v.step) % (unsigned)v.audit_stride == 0;
+        }
+        // wavefront-aggregated append of the cells the plain integrator must see
+        const unsigned long long need = __ballot(fallback || audit);
+        n_used += (unsigned)__popcll(__ballot(mine && !fallback));
+        n_fb += (unsigned)__popcll(__ballot(fallback));
+        if (need) {
+            unsigned slot0 = 0;
+            if (lane == 0) slot0 = atomicAdd(count, (unsigned)__popcll(need));
+            slot0 = __shfl(slot0, 0);
+            if (fallback || audit) {
+                const unsigned below = (unsigned)__popcll(need & ((1ull << lane) - 1ull));
+                list[slot0 + below] = (unsigned)c | (audit ? CHEM_AUDIT : 0u);
+            }
+        }
     }
-    // wavefront-aggregated append of the cells the plain integrator must see
-    const unsigned long long need = __ballot(fallback || audit);
-    const unsigned used = (unsigned)__popcll(__ballot(mine && !fallback));
-    const unsigned fb = (unsigned)__popcll(__ballot(fallback));
-    unsigned slot0 = 0;
     if (lane == 0) {
-        if (need) slot0 = atomicAdd(count, (unsigned)__popcll(need));
-        if (used) atomicAdd(&blk_used, used);
-        if (fb) atomicAdd(&blk_fb, fb);
-    }
-    slot0 = __shfl(slot0, 0);
-    if (fallback || audit) {
-        const unsigned below = (unsigned)__popcll(need & ((1ull << lane) - 1ull));
-        list[slot0 + below] = (unsigned)c | (audit ? CHEM_AUDIT : 0u);
+        if (n_used) atomicAdd(&blk_used, n_used);
+        if (n_fb) atomicAdd(&blk_fb, n_fb);
     }
     __syncthreads();
     if (threadIdx.x == 0) {  // one update per block
@@ -509,7 +584,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc_sur_decode(MultiView<P> v, const f
 }
 
 template <typename P>
-__global__ __launch_bounds__(BLOCK) void k_mc_chem_list(MultiView<P> v, const unsigned* list, const unsigned* count)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CHEM_WAVES, 8))) void k_mc_chem_list(MultiView<P> v, const unsigned* list, const unsigned* count)
 {
     using namespace sur;
     const unsigned total = *count;
@@ -581,8 +656,8 @@ __device__ __forceinline__ void mixture_rates(const MultiView<P>& v, int c, doub
     const double cp = v.u.cp(cp_mass(Tsi, Y0));
     const double mu = v.u.mu(mu_si);
     const double kap = v.u.thermal_conductivity(kap_si);
-    v.omix[c] = 2 * p * 1 / (p * 1 + 2 * mu);
-    v.omix[v.d.n + c] = 2 * p * cp * 1 / (p * cp * 1 + 2 * kap);
+    v.omix[c] = quot(2 * p * 1, p * 1 + 2 * mu);
+    v.omix[v.d.n + c] = quot(2 * p * cp * 1, p * cp * 1 + 2 * kap);
 }
 
 // The transport pass of the FP32 path, all in binary32: species
@@ -597,7 +672,7 @@ __device__ __forceinline__ void species_transport_fp32(const MultiView<P>& v, in
     double* const* Fd = v.fld;
     const double rho = Fd[LBM_FIELD_RHO][c], T = Fd[LBM_FIELD_T][c];
     const float p = (float)Fd[LBM_FIELD_P][c];
-    const double irho = 1.0 / rho;
+    const double irho = quot(1.0, rho);
     float ra[NS], Xa[NS];
     double Y0[NS];
 #pragma unroll
@@ -680,43 +755,44 @@ __global__ __launch_bounds__(BLOCK) void k_mc_species_transport(MultiView<P> v)
     double* const* Fd = v.fld;
     const double rho = Fd[LBM_FIELD_RHO][c], T = Fd[LBM_FIELD_T][c], p = Fd[LBM_FIELD_P][c];
     double ra[NS], Xa[NS], Y0[NS];
+    const Divisor drho = divisor(rho);
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
         ra[a] = v.rhoa[a * n + c];
         Xa[a] = v.X[a * n + c];
-        Y0[a] = ra[a] / rho;
+        Y0[a] = quot(ra[a], drho);
     }
     normalize(Y0);
     const double Tsi = v.u.si_temp(T);
     const double rho_si = v.u.si_rho(rho);
-    // species viscosities and Wilke weights at (T, rho); transport arithmetic
-    // R is binary64 on the plain path and binary32 on the FP32 path
-    using R = typename std::conditional<sizeof(P) == 4, float, double>::type;
+    // species viscosities and Wilke weights at (T, rho)
     const double lnT = log(Tsi);
-    const R lnTr = (R)lnT;
-    R mu[NS], den[NS];
+    double mu[NS], den[NS];
+    Divisor dmu[NS];
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
-        mu[a] = species_viscosity_r<R>(a, lnTr);
+        mu[a] = species_viscosity(a, lnT);
+        dmu[a] = divisor(mu[a]);
         den[a] = 0;
     }
 #pragma unroll
-    for (int a = 0; a < NS; ++a)
+    for (int a = 0; a < NS; ++a) {
+        den[a] += Xa[a];  // Phi_aa = 1
 #pragma unroll
-        for (int b = a; b < NS; ++b) {
-            const R f1 = R(1) + sqrt(mu[a] / mu[b]) * (R)sqrt(sqrt(W[b] / W[a]));
-            const R pab = f1 * f1 / (R)sqrt(8.0 * (1.0 + W[a] / W[b]));
-            den[a] += (R)Xa[b] * pab;
-            if (b != a) den[b] += (R)Xa[a] * (mu[b] / mu[a] * (R)W[a] / (R)W[b] * pab);
+        for (int b = a + 1; b < NS; ++b) {
+            const double f1 = 1.0 + sqrt(quot(mu[a], dmu[b])) * sqrt(sqrt(W[b] / W[a]));
+            const double pab = quot(f1 * f1, wilke_divisor(a, b));
+            den[a] += Xa[b] * pab;
+            den[b] += Xa[a] * (over_w(quot(mu[b], dmu[a]) * W[a], b) * pab);
         }
+    }
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
-        const double visc = Xa[a] * (double)v.u.mu(mu[a]) / (double)den[a];
-        v.tsp[a * n + c] = P(2 * Xa[a] * p / (Xa[a] * p + 2 * visc));
+        const double visc = quot(Xa[a] * (double)v.u.mu(mu[a]), den[a]);
+        v.tsp[a * n + c] = P(quot(2 * Xa[a] * p, Xa[a] * p + 2 * visc));
     }
 
-    const double p_si = pressure(Tsi, rho_si, Y0);
-    const R p_sir = (R)p_si;
+    const Divisor dp_si = divisor(pressure(Tsi, rho_si, Y0));
     // Maxwell-Stefan friction with the binary diffusivities of the state.  The
     // fit table is symmetric, so D_ab = D_ba is evaluated once per pair; the
     // b = a term, k (u_a - u_a), is zero and skipped.  Each acc[a] still sums
@@ -733,9 +809,9 @@ __global__ __launch_bounds__(BLOCK) void k_mc_species_transport(MultiView<P> v)
     for (int a = 0; a < NS; ++a)
 #pragma unroll
         for (int b = a + 1; b < NS; ++b) {
-            const double D = v.u.nu(binary_diff_r<R>(a, b, lnTr, p_sir));
-            const double kab = -1.0 * p * Xa[a] * Xa[b] / D;
-            const double kba = -1.0 * p * Xa[b] * Xa[a] / D;
+            const Divisor D = divisor(v.u.nu(quot(exp(poly4(DIFF_FIT[a][b], lnT)), dp_si)));
+            const double kab = quot(-1.0 * p * Xa[a] * Xa[b], D);
+            const double kba = quot(-1.0 * p * Xa[b] * Xa[a], D);
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 acc[a][d] += kab * (ua[d][a] - ua[d][b]);
@@ -743,9 +819,11 @@ __global__ __launch_bounds__(BLOCK) void k_mc_species_transport(MultiView<P> v)
             }
         }
 #pragma unroll
-    for (int a = 0; a < NS; ++a)
+    for (int a = 0; a < NS; ++a) {
+        const Divisor dra = divisor(ra[a]);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) v.tsp[((1 + d) * NS + a) * n + c] = P(acc[a][d] * 1.0 / ra[a]);
+        for (int d = 0; d < 3; ++d) v.tsp[((1 + d) * NS + a) * n + c] = P(quot(acc[a][d] * 1.0, dra));
+    }
 }
 
 // Collide_Species of species a at cell c (lbm-collision.cpp:452-520) from
@@ -780,9 +858,10 @@ __device__ __forceinline__ void species_collision(const MultiView<P>& v, int c, 
     }
     // FP32 path: one reciprocal for the three divisions
     constexpr bool FAST = sizeof(P) == 4;
-    const double ira = FAST ? 1.0 / ra : 0.0;
-    const double uraw[3] = {FAST ? mom[0] * ira : mom[0] / ra, FAST ? mom[1] * ira : mom[1] / ra,
-                            FAST ? mom[2] * ira : mom[2] / ra};
+    const Divisor dra = divisor(ra);
+    const double ira = FAST ? quot(1.0, dra) : 0.0;
+    const double uraw[3] = {FAST ? mom[0] * ira : quot(mom[0], dra), FAST ? mom[1] * ira : quot(mom[1], dra),
+                            FAST ? mom[2] * ira : quot(mom[2], dra)};
     const double udu[3] = {uraw[0] + Fa[0], uraw[1] + Fa[1], uraw[2] + Fa[2]};
     const double Ra = v.u.cp(R_UNIV / W[a]);
     const double theta = Ra * T;
@@ -798,7 +877,7 @@ __device__ __forceinline__ void species_collision(const MultiView<P>& v, int c, 
     }
     double corr[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) corr[d] = 1 * (2.0 - om) / (2.0 * ra * om) * dQ[d];
+    for (int d = 0; d < 3; ++d) corr[d] = quot(1 * (2.0 - om), 2.0 * ra * om) * dQ[d];
     Axis3<double> Fe[3], Fu[3];
     feq_axes<double>(Fe, uraw, theta, corr);
     feq_axes<double>(Fu, udu, theta, corr);
@@ -1037,8 +1116,11 @@ __global__ __launch_bounds__(BLOCK) void k_mc_side_push_aa(MultiView<P> v)
 // forms do the same arithmetic in the same order.
 enum : int { OMIX_OM = 0, OMIX_OM1 = 1, OMIX_THETA = 2, OMIX_USHIFT = 3, OMIX_DQ = 4, OMIX_PLANES = 7 };
 
+// The FP64 form holds 174 VGPRs by itself; three waves (168, 28 B of scratch)
+// took 284 us against 317 with two on 128x96x48 cells.
 template <typename P, int PART>
-__global__ __launch_bounds__(BLOCK) void k_mc_collide(MultiView<P> v)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(P) == 8 && PART == 0 && NS <= 16 ? 3 : 1, 8)))
+void k_mc_collide(MultiView<P> v)
 {
     const int c = blockIdx.x * BLOCK + threadIdx.x;
     bool warn = false;
@@ -1074,18 +1156,20 @@ __global__ __launch_bounds__(BLOCK) void k_mc_collide(MultiView<P> v)
         const double vel[3] = {Fd[LBM_FIELD_U][c], Fd[LBM_FIELD_V][c], Fd[LBM_FIELD_W][c]};
         // FP32: products with reciprocals in place of divisions
         constexpr bool FAST = sizeof(P) == 4;
-        const double irho = 1.0 / rho;
+        const Divisor drho = divisor(rho);
+        const double irho = quot(1.0, drho);
         double ra[NS], Y0[NS], X0[NS];
 #pragma unroll
         for (int a = 0; a < NS; ++a) {
             ra[a] = v.rhoa[a * n + c];
-            Y0[a] = FAST ? ra[a] * irho : ra[a] / rho;
+            Y0[a] = FAST ? ra[a] * irho : quot(ra[a], drho);
         }
         normalize(Y0);
         const double Tsi = v.u.si_temp(T);
         const double Wm = mean_W(Y0);
-        const double Rmix = v.u.cp(R_UNIV / Wm);
-        const double theta = v.u.energy_mass(R_UNIV * Tsi / Wm);
+        const Divisor dWm = divisor(Wm);
+        const double Rmix = v.u.cp(quot(R_UNIV, dWm));
+        const double theta = v.u.energy_mass(quot(R_UNIV * Tsi, dWm));
         double om, om1;
         if constexpr (PART == 1) {
             om = v.omix[OMIX_OM * n + c];
@@ -1098,15 +1182,18 @@ __global__ __launch_bounds__(BLOCK) void k_mc_collide(MultiView<P> v)
             using R = typename std::conditional<sizeof(P) == 4, float, double>::type;
             const double mu = v.u.mu(mix_viscosity_r<R>((R)lnT, X0));
             const double kap = v.u.thermal_conductivity(mix_conductivity_r<R>((R)lnT, X0));
-            om1 = 2 * p * cp * 1 / (p * cp * 1 + 2 * kap);
-            om = 2 * p * 1 / (p * 1 + 2 * mu);
+            om1 = quot(2 * p * cp * 1, p * cp * 1 + 2 * kap);
+            om = quot(2 * p * 1, p * 1 + 2 * mu);
         }
-        warn = (1 / om <= 0.5) || (1 / om1 <= 0.5);
-        double Uint = Fd[LBM_FIELD_RHOE][c] / rho;
+        warn = (quot(1.0, om) <= 0.5) || (quot(1.0, om1) <= 0.5);
+        double Uint = quot(Fd[LBM_FIELD_RHOE][c], drho);
+        // (both species loops stay rolled: unrolled they hold 256 VGPRs, one wave
+        // per SIMD fewer)
+#pragma unroll 1
         for (int a = 0; a < NS; ++a) {
             const double ux = v.ua[(0 * NS + a) * n + c], uy = v.ua[(1 * NS + a) * n + c],
                          uz = v.ua[(2 * NS + a) * n + c];
-            Uint = Uint - (FAST ? 0.5 * ra[a] * irho : 0.5 * ra[a] / rho) * (ux * ux + uy * uy + uz * uz);
+            Uint = Uint - (FAST ? 0.5 * ra[a] * irho : quot(0.5 * ra[a], drho)) * (ux * ux + uy * uy + uz * uz);
         }
         const int nm[3] = {cell(v.d, x.i - 1, x.j, x.k), cell(v.d, x.i, x.j - 1, x.k), c - 1};
         const int np[3] = {cell(v.d, x.i + 1, x.j, x.k), cell(v.d, x.i, x.j + 1, x.k), c + 1};
@@ -1116,20 +1203,22 @@ __global__ __launch_bounds__(BLOCK) void k_mc_collide(MultiView<P> v)
         double irn[3], irp[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            irn[d] = 1.0 / Fd[LBM_FIELD_RHO][nm[d]];
-            irp[d] = 1.0 / Fd[LBM_FIELD_RHO][np[d]];
+            irn[d] = quot(1.0, Fd[LBM_FIELD_RHO][nm[d]]);
+            irp[d] = quot(1.0, Fd[LBM_FIELD_RHO][np[d]]);
         }
-        const double invT = 1.0 / Tsi;
+        const double invT = quot(1.0, Tsi);
+        const double om_ratio = quot(om1, -om + om1), om_half = quot(0.5 * (2.0 - om1), -om + om1);
+#pragma unroll 1
         for (int a = 0; a < NS; ++a) {
             const double ha = v.u.energy_mass((FAST ? h_RT_inv(a, Tsi, invT) : h_RT(a, Tsi)) * R_UNIV * Tsi * inv_w(a));
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 const double uad = v.ua[(d * NS + a) * n + c];
-                qdiff[d] += om1 / (-om + om1) * ha * ra[a] * (uad - vel[d]);
+                qdiff[d] += om_ratio * ha * ra[a] * (uad - vel[d]);
                 const double Yn = v.rhoa[a * n + nm[d]] * irn[d];
                 const double Yp = v.rhoa[a * n + np[d]] * irp[d];
                 const double dY = fd_fuw<double>(Yn, ra[a] * irho, Yp, uad - vel[d], v.type[nm[d]], v.type[np[d]]);
-                qcorr[d] += 0.5 * (2.0 - om1) / (-om + om1) * 1 * p * ha * dY;
+                qcorr[d] += om_half * 1 * p * ha * dY;
             }
         }
         // mixture gas constant of a neighbour, R_univ sum(Y/W) / sum(Y): the
@@ -1143,7 +1232,7 @@ __global__ __launch_bounds__(BLOCK) void k_mc_collide(MultiView<P> v)
                 sYW += ra_m * inv_w(a);
                 sY += ra_m;
             }
-            return v.u.cp(R_UNIV * sYW / sY);
+            return v.u.cp(quot(R_UNIV * sYW, sY));
         };
         double dQ[3];
 #pragma unroll
@@ -1360,44 +1449,45 @@ __device__ inline void cholesky_solve3(double A[NS][NS], double B[NS][3])
 }
 
 // The same solve with A held as its lower triangle, L[tri(i, j)] = A[i][j]
-// for j <= i (36 fewer live doubles); same operations in the same order.
+// for j <= i (36 fewer live doubles); same operations in the same order, the
+// quotients of a pivot through its one reciprocal (the 90 divisions by 9
+// pivots were a third of the FP64 moment pass's operations).
 constexpr int NTRI = NS * (NS + 1) / 2;
 __host__ __device__ constexpr int tri(int i, int j) { return i * (i + 1) / 2 + j; }
 
-// (T = double: the FP64 path; T = float: the FP32 path's binary32 solve.)
-template <typename T>
-__device__ inline void cholesky_solve3(T L[NTRI], T B[NS][3])
+__device__ inline void cholesky_solve3(double L[NTRI], double B[NS][3])
 {
+    Divisor piv[NS];
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-        T s = L[tri(j, j)];
+        double s = L[tri(j, j)];
 #pragma unroll
         for (int k = 0; k < j; ++k) s -= L[tri(j, k)] * L[tri(j, k)];
-        const T d = sqrt(s);
-        L[tri(j, j)] = d;
+        const double d = sqrt(s);
+        piv[j] = divisor(d);
 #pragma unroll
         for (int i = j + 1; i < NS; ++i) {
-            T t = L[tri(i, j)];
+            double t = L[tri(i, j)];
 #pragma unroll
             for (int k = 0; k < j; ++k) t -= L[tri(i, k)] * L[tri(j, k)];
-            L[tri(i, j)] = t / d;
+            L[tri(i, j)] = quot(t, piv[j]);
         }
     }
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
-            T t = B[i][r];
+            double t = B[i][r];
 #pragma unroll
             for (int k = 0; k < i; ++k) t -= L[tri(i, k)] * B[k][r];
-            B[i][r] = t / L[tri(i, i)];
+            B[i][r] = quot(t, piv[i]);
         }
 #pragma unroll
         for (int i = NS - 1; i >= 0; --i) {
-            T t = B[i][r];
+            double t = B[i][r];
 #pragma unroll
             for (int k = i + 1; k < NS; ++k) t -= L[tri(k, i)] * B[k][r];
-            B[i][r] = t / L[tri(i, i)];
+            B[i][r] = quot(t, piv[i]);
         }
     }
 }
@@ -1474,11 +1564,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(P)
     const double rho_old_si = v.u.si_rho(rho_old);
     const double p_old = Fd[LBM_FIELD_P][c];
     constexpr bool FAST = sizeof(P) == 4;  // FP32: reciprocals in place of divisions
-    const double irho_old = 1.0 / rho_old;
+    const Divisor drho_old = divisor(rho_old);
+    const double irho_old = quot(1.0, drho_old);
     double Yold[NS], Xold[NS];
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
-        Yold[a] = FAST ? v.rhoa[a * n + c] * irho_old : v.rhoa[a * n + c] / rho_old;
+        Yold[a] = FAST ? v.rhoa[a * n + c] * irho_old : quot(v.rhoa[a * n + c], drho_old);
         Xold[a] = v.X[a * n + c];
     }
     normalize(Yold);
@@ -1536,12 +1627,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(P)
         m1 += my;
         m2 += mz;
     }
-    const double vel[3] = {m0 / rho, m1 / rho, m2 / rho};
+    const Divisor drho = divisor(rho);
+    const double vel[3] = {quot(m0, drho), quot(m1, drho), quot(m2, drho)};
     // Maxwell-Stefan velocities: A u = (rho u)_a with the old state's D, p, X;
     // then the internal energy U = rho e / rho - sum 1/2 rho_a |u_a|^2 / rho and
     // the species velocities are written (not live across the T iteration)
-    double Uint = re / rho;
+    double Uint = quot(re, drho);
     if constexpr (sizeof(P) == 8) {
+        const Divisor dp_old = divisor(p_old_si);
         double A[NTRI];  // lower triangle; A[a][b] = A[b][a] = A[tri(max, min)]
 #pragma unroll
         for (int a = 0; a < NS; ++a)
@@ -1551,8 +1644,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(P)
                 if (b == a) {
                     A[tri(a, a)] = rr[a] == 0.0 ? 1.0 : rr[a];
                 } else {
-                    const double D = v.u.nu(binary_diff(a, b, lnT_old, p_old_si));
-                    A[tri(b, a)] = -1.0 * 1 / 2.0 * p_old * Xold[a] * Xold[b] / D;
+                    const double D = v.u.nu(quot(exp(poly4(DIFF_FIT[a][b], lnT_old)), dp_old));
+                    A[tri(b, a)] = quot(-1.0 * 1 / 2.0 * p_old * Xold[a] * Xold[b], D);
                 }
             }
 #pragma unroll
@@ -1591,7 +1684,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(P)
             for (int d = 0; d < 3; ++d) Bf[a][d] = s_B[3 * a + d][threadIdx.x];
         }
         cholesky_solve3_rcp(A, Bf);
-        const double irho = 1.0 / rho;
+        const double irho = quot(1.0, drho);
 #pragma unroll
         for (int a = 0; a < NS; ++a) {
             const double b0 = Bf[a][0], b1 = Bf[a][1], b2 = Bf[a][2];
@@ -1604,13 +1697,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(P)
     }
     // temperature from energy at the new composition
     double Y[NS], X[NS];
-    const double irho_new = 1.0 / rho;
+    const double irho_new = quot(1.0, drho);
 #pragma unroll
-    for (int a = 0; a < NS; ++a) Y[a] = FAST ? rr[a] * irho_new : rr[a] / rho;
+    for (int a = 0; a < NS; ++a) Y[a] = FAST ? rr[a] * irho_new : quot(rr[a], drho);
     normalize(Y);
     if constexpr (sizeof(P) == 8) {  // (write order measured fastest at one wave per SIMD)
         for (int a = 0; a < NS; ++a)
-            Uint = Uint - 0.5 * rr[a] / rho * (B[a][0] * B[a][0] + B[a][1] * B[a][1] + B[a][2] * B[a][2]);
+            Uint = Uint - quot(0.5 * rr[a], drho) * (B[a][0] * B[a][0] + B[a][1] * B[a][1] + B[a][2] * B[a][2]);
         const double usi = v.u.si_energy_mass(Uint);
         const double rho_si = v.u.si_rho(rho);
         const double Tsi = T_from_UV(usi, Y, Tsi_old);
@@ -1771,9 +1864,10 @@ __device__ inline void cell_vals(const MultiView<P>& v, int c, double out[NV])
     out[2] = v.fld[LBM_FIELD_V][c];
     out[3] = v.fld[LBM_FIELD_W][c];
     const double r = v.fld[LBM_FIELD_RHO][c];
+    const Divisor dr = divisor(r);
     out[4] = r;
 #pragma unroll
-    for (int a = 0; a < NS; ++a) out[5 + a] = v.rhoa[a * n + c] / r;
+    for (int a = 0; a < NS; ++a) out[5 + a] = quot(v.rhoa[a * n + c], dr);
 }
 
 // one-sided second order into the domain (normal_derivative) or the
@@ -2603,6 +2697,16 @@ void launch_mc(McKernel k, const MultiView<P>& v, hipStream_t s)
         switch (k) {
         case McKernel::Init: hipLaunchKernelGGL(k_mc_init<P>, grid1(v.d.n), dim3(BLOCK), 0, s, v); break;
         case McKernel::Chemistry: hipLaunchKernelGGL(k_mc_chemistry<P>, grid1(v.d.n), dim3(BLOCK), 0, s, v); break;
+        case McKernel::ChemistryBeside:
+            // Beside the transport pass and the mixture collide: more than half a
+            // CU's LDS per block keeps one block, a wavefront per SIMD, on each CU
+            // and leaves the rest of its registers to the other stream, whose
+            // kernels wait on loads.  Unlimited, the chemistry takes every
+            // register first and the two run one after the other: a step of
+            // 131x97x75 cells FP32 1.651 -> 1.597 ms, 128x96x48 FP64 1.960 ->
+            // 1.930 (two blocks: 1.650, 1.946).
+            hipLaunchKernelGGL(k_mc_chemistry<P>, grid1(v.d.n), dim3(BLOCK), 96 * 1024, s, v);
+            break;
         case McKernel::SpeciesTransport:
             hipLaunchKernelGGL(k_mc_species_transport<P>, dim3(xcd_grid(v.d.n, BLOCK)), dim3(BLOCK), 0, s, v);
             break;
@@ -2756,16 +2860,17 @@ void launch_mc_aa_collide(const MultiView<P>& v, int a0, int na, bool side, hipS
 
 
 template <typename P>
-void launch_mc_sur_chemistry(const MultiView<P>& v, const sur::Mlp& net, uint16_t* X, float* Y, uint8_t* flag,
-                             int64_t rows, unsigned* list, unsigned* count, hipStream_t s)
+void launch_mc_sur_chemistry(const MultiView<P>& v, const sur::Mlp& net, unsigned* list, unsigned* count,
+                             hipStream_t s)
 {
     if constexpr (!kernels_built<P>() || !sur::ENABLED) {
         return;  // refused before launch (lbm_create, surrogate entry points)
     } else {
         hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, count);
-        hipLaunchKernelGGL(k_mc_sur_features<P>, grid1(v.d.n), dim3(BLOCK), 0, s, v, X, flag);
-        sur::mlp_infer_bf16(net, X, rows, Y, s);
-        hipLaunchKernelGGL(k_mc_sur_decode<P>, grid1(v.d.n), dim3(BLOCK), 0, s, v, Y, flag, list, count);
+        const int64_t nb = (v.d.n + SUR_WAVES * 64 - 1) / (SUR_WAVES * 64);
+        const int cus = cu_count();
+        hipLaunchKernelGGL(k_mc_surrogate<P>, dim3((unsigned)(nb < cus ? nb : cus)), dim3(SUR_WAVES * 64), 0, s, v, net,
+                           list, count);
     }
 }
 
@@ -2790,11 +2895,11 @@ template void launch_mc_aa_save<float>(const MultiView<float>&, bool, int, int, 
 template void launch_mc_aa_collide<double>(const MultiView<double>&, int, int, bool, hipStream_t);
 template void launch_mc_aa_collide<float>(const MultiView<float>&, int, int, bool, hipStream_t);
 template void launch_mc_tms<float>(const MultiView<float>&, const int*, const int*, int, double*, hipStream_t);
-template void launch_mc_sur_chemistry<float>(const MultiView<float>&, const sur::Mlp&, uint16_t*, float*,
-                                             uint8_t*, int64_t, unsigned*, unsigned*, hipStream_t);
+template void launch_mc_sur_chemistry<float>(const MultiView<float>&, const sur::Mlp&, unsigned*, unsigned*,
+                                             hipStream_t);
 template void launch_mc_chem_list<float>(const MultiView<float>&, const unsigned*, const unsigned*, hipStream_t);
-template void launch_mc_sur_chemistry<double>(const MultiView<double>&, const sur::Mlp&, uint16_t*, float*,
-                                              uint8_t*, int64_t, unsigned*, unsigned*, hipStream_t);
+template void launch_mc_sur_chemistry<double>(const MultiView<double>&, const sur::Mlp&, unsigned*, unsigned*,
+                                              hipStream_t);
 template void launch_mc_chem_list<double>(const MultiView<double>&, const unsigned*, const unsigned*, hipStream_t);
 template void launch_mc_tms<double>(const MultiView<double>&, const int*, const int*, int, double*, hipStream_t);
 template void launch_mc_tms_in<double>(const MultiView<double>&, const int*, const int*, int, hipStream_t);

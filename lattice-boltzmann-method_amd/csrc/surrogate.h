@@ -70,9 +70,6 @@ void next_iteration(int* it, hipStream_t s);
 // In-step style inference: Y [M][16] FP32 from normalised X [M][16] FP32 (any
 // M), activations in registers, weights staged in LDS.
 void mlp_infer(const Mlp& net, const float* X, int M, float* Y, hipStream_t s);
-// The same network on BF16 inputs X [rows][16] (rows a multiple of 256) into
-// FP32 outputs Y [rows][16], weights staged in LDS.
-void mlp_infer_bf16(const Mlp& net, const uint16_t* X, int64_t rows, float* Y, hipStream_t s);
 // Column statistics of `rows` capture rows into `stats` [SS_SIZE] (device);
 // `part` holds STATS_BLOCKS * 32 * 4 doubles.  envelope_only: only the
 // envelope (SS_LO, SS_HI) is rewritten, the normalisation kept.

@@ -238,7 +238,11 @@ __global__ __launch_bounds__(512) void k_mlp_infer(Mlp net, const float* X, int 
             xin[wave][i] = f2bf(row < M ? X[(size_t)row * 16 + (i % 16)] : 0.f);
         }
         __syncthreads();
-        mlp_rows32(Wf, bias, xin[wave], yout[wave]);
+        const v4s x[2] = {input_frag(xin[wave], 0), input_frag(xin[wave], 1)};
+        v4f y[2];
+        mlp_rows32(Wf, bias, x, y);
+        output_frag(yout[wave], 0, y[0]);
+        output_frag(yout[wave], 1, y[1]);
         __syncthreads();
         for (int i = lane; i < 32 * 16; i += 64) {
             const int row = base + wave * 32 + i / 16;
@@ -258,33 +262,6 @@ int infer_grid(int M)
 void mlp_infer(const Mlp& net, const float* X, int M, float* Y, hipStream_t s)
 {
     hipLaunchKernelGGL(k_mlp_infer, dim3(infer_grid(M)), dim3(512), 0, s, net, X, M, Y);
-}
-
-// In-step network pass: inputs already BF16 in HBM, 8 wavefronts x 32 rows
-// per pass of a 512-thread block, grid-stride; rows is a multiple of 256.
-__global__ __launch_bounds__(512) void k_mlp_rows(Mlp net, const uint16_t* X, int64_t rows, float* Y)
-{
-    __shared__ __align__(16) uint16_t Wf[FRAG_TOTAL];
-    __shared__ float bias[BIAS_TOTAL];
-    stage_net(net, Wf, bias);
-    __syncthreads();
-    const int wave = threadIdx.x >> 6;
-    for (int64_t base = (int64_t)blockIdx.x * IROWS; base < rows; base += (int64_t)gridDim.x * IROWS) {
-        // keeps the weight fragments' LDS reads inside the loop (hoisted out
-        // of it they would need 576 registers)
-        asm volatile("" ::: "memory");
-        const int64_t r0 = base + wave * 32;
-        mlp_rows32(Wf, bias, X + r0 * 16, Y + r0 * 16);
-    }
-}
-
-void mlp_infer_bf16(const Mlp& net, const uint16_t* X, int64_t rows, float* Y, hipStream_t s)
-{
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const int64_t groups = rows / IROWS;
-    const int grid = (int)(groups < 2 * cus ? (groups > 0 ? groups : 1) : 2 * cus);
-    hipLaunchKernelGGL(k_mlp_rows, dim3(grid), dim3(512), 0, s, net, X, rows, Y);
 }
 
 // ---------------------------------------------------- training data

@@ -140,69 +140,82 @@ __device__ __forceinline__ v4s act_frag(const v4f z)
 }
 
 // Evaluates the network for 32 rows (two batch tiles) held by one wavefront.
-// `Wf` and `bias` are the fragment-ordered weights and the biases (LDS), `xin`
-// the BF16 inputs [32][16] of this wavefront and `yout` its FP32 outputs
-// [32][16] (LDS or global; 16-byte aligned).  Each accumulator starts from
-// the layer's bias.
-__device__ __forceinline__ void mlp_rows32(const uint16_t* Wf, const float* bias, const uint16_t* xin, float* yout)
+// `Wf` and `bias` are the fragment-ordered weights and the biases (LDS), x[bt]
+// the BF16 inputs of batch tile bt (row lane % 16, features 4 (lane / 16) +
+// 0..3), out[bt] its FP32 outputs in the same places.  Each accumulator
+// starts from the layer's bias.
+//
+// Bound by the activations (5 vector operations, an exp2 and a reciprocal each:
+// two thirds of the pass).  Output tile t + 1 is multiplied while tile t goes
+// through its activation: the two are independent, so the matrix
+// instructions and the LDS reads of their weights run under the activations
+// instead of ahead of them.
+constexpr int HTILES = 128 / 16, KSTEPS = 128 / 32;
+struct Acc2 {
+    v4f c[2];
+};
+template <int L>
+__device__ __forceinline__ Acc2 hidden_tile(const uint16_t* Wf, const float* bias, const v4s act[2][HTILES], int t,
+                                            int lane)
+{
+    const uint16_t* W = Wf + frag_offset(L);
+    Acc2 a;
+    a.c[0] = a.c[1] = bias_frag(bias + bias_offset(L), 16 * t, lane);
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) {
+        const v8bf w = load_frag8(W + ((t * KSTEPS + s) * 64 + lane) * 8);
+#pragma unroll
+        for (int bt = 0; bt < 2; ++bt)
+            a.c[bt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, pair_frag(act[bt][2 * s], act[bt][2 * s + 1]), a.c[bt],
+                                                             0, 0, 0);
+    }
+    return a;
+}
+__device__ __forceinline__ Acc2 input_tile(const uint16_t* Wf, const float* bias, const v4s x[2], int t, int lane)
+{
+    const v4s w = load_frag(Wf + frag_offset(0) + (t * 64 + lane) * 4);
+    const v4f b = bias_frag(bias + bias_offset(0), 16 * t, lane);
+    Acc2 a;
+#pragma unroll
+    for (int bt = 0; bt < 2; ++bt) a.c[bt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w, x[bt], b, 0, 0, 0);
+    return a;
+}
+// `next(t)` multiplies tile t of a layer; to[bt][t] receives its activations.
+template <typename Next>
+__device__ __forceinline__ void layer_tiles(Next next, v4s to[2][HTILES])
+{
+    Acc2 a = next(0);
+#pragma unroll
+    for (int t = 0; t < HTILES; ++t) {
+        Acc2 b = a;
+        if (t + 1 < HTILES) b = next(t + 1);
+        to[0][t] = act_frag(a.c[0]);
+        to[1][t] = act_frag(a.c[1]);
+        a = b;
+    }
+}
+__device__ __forceinline__ void mlp_rows32(const uint16_t* Wf, const float* bias, const v4s x[2], v4f out[2])
 {
     const int lane = threadIdx.x & 63;
-    const int r = lane & 15, kq = (lane >> 4) * 4;
-    constexpr int H = 128 / 16;  // hidden tiles
-    v4s act[2][H], nxt[2][H];
-    // layer 0: K = 16, one K-step
-    {
-        const uint16_t* W0 = Wf + frag_offset(0);
-        v4s x[2];
-#pragma unroll
-        for (int bt = 0; bt < 2; ++bt) x[bt] = load_frag(xin + (bt * 16 + r) * 16 + kq);
-#pragma unroll
-        for (int t = 0; t < H; ++t) {
-            const v4s a = load_frag(W0 + (t * 64 + lane) * 4);
-            const v4f b = bias_frag(bias + bias_offset(0), 16 * t, lane);
-#pragma unroll
-            for (int bt = 0; bt < 2; ++bt)
-                act[bt][t] = act_frag(__builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, x[bt], b, 0, 0, 0));
-        }
-    }
-    // layers 1 and 2: 128 -> 128, 32-deep K-steps
-    constexpr int KS = 128 / 32;
-#pragma unroll
-    for (int L = 1; L <= 2; ++L) {
-        const uint16_t* WL = Wf + frag_offset(L);
-        const float* bL = bias + bias_offset(L);
-#pragma unroll
-        for (int t = 0; t < H; ++t) {
-            v4f acc0 = bias_frag(bL, 16 * t, lane), acc1 = acc0;
-#pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                const v8bf a = load_frag8(WL + ((t * KS + s) * 64 + lane) * 8);
-                acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pair_frag(act[0][2 * s], act[0][2 * s + 1]), acc0,
-                                                                0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pair_frag(act[1][2 * s], act[1][2 * s + 1]), acc1,
-                                                                0, 0, 0);
-            }
-            nxt[0][t] = act_frag(acc0);
-            nxt[1][t] = act_frag(acc1);
-        }
-#pragma unroll
-        for (int t = 0; t < H; ++t) {
-            act[0][t] = nxt[0][t];
-            act[1][t] = nxt[1][t];
-        }
-    }
-    // layer 3: 128 -> 16, no activation
-    const uint16_t* W3 = Wf + frag_offset(3);
-    const float* b3 = bias + bias_offset(3);
-    v4f acc0 = bias_frag(b3, 0, lane), acc1 = acc0;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        const v8bf a = load_frag8(W3 + (s * 64 + lane) * 8);
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pair_frag(act[0][2 * s], act[0][2 * s + 1]), acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pair_frag(act[1][2 * s], act[1][2 * s + 1]), acc1, 0, 0, 0);
-    }
-    *reinterpret_cast<v4f*>(yout + r * 16 + kq) = acc0;
-    *reinterpret_cast<v4f*>(yout + (16 + r) * 16 + kq) = acc1;
+    v4s h0[2][HTILES], h1[2][HTILES];
+    layer_tiles([&](int t) { return input_tile(Wf, bias, x, t, lane); }, h0);
+    layer_tiles([&](int t) { return hidden_tile<1>(Wf, bias, h0, t, lane); }, h1);
+    layer_tiles([&](int t) { return hidden_tile<2>(Wf, bias, h1, t, lane); }, h0);
+    const Acc2 a = hidden_tile<3>(Wf, bias, h0, 0, lane);  // 128 -> 16, no activation
+    out[0] = a.c[0];
+    out[1] = a.c[1];
+}
+// The inputs of batch tile bt from BF16 rows [..][16] in LDS.
+__device__ __forceinline__ v4s input_frag(const uint16_t* xin, int bt)
+{
+    const int lane = threadIdx.x & 63;
+    return load_frag(xin + (bt * 16 + (lane & 15)) * 16 + (lane >> 4) * 4);
+}
+// The outputs of batch tile bt into FP32 rows [..][16] in LDS.
+__device__ __forceinline__ void output_frag(float* yout, int bt, const v4f o)
+{
+    const int lane = threadIdx.x & 63;
+    *reinterpret_cast<v4f*>(yout + (bt * 16 + (lane & 15)) * 16 + (lane >> 4) * 4) = o;
 }
 
 // Stages the fragment-ordered weights and biases of `net` into LDS.
