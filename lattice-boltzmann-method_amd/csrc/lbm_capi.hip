@@ -5,11 +5,13 @@
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cstdlib>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "lbm_amd.h"
@@ -22,6 +24,19 @@ using namespace lbm;
 namespace {
 
 thread_local std::string g_create_error;
+
+// Pinned staging of large downloads, allocated at a context's first one.
+// 2 slots for each of 8 copying threads; a chunk is long enough that the
+// bus runs at its rate and short enough that the first copy starts early.
+struct Stage {
+    static constexpr int WORKERS = 8, SLOTS = 2 * WORKERS;
+    static constexpr size_t CHUNK = (size_t)1 << 20;
+    // below this the copy through the runtime's own staging takes about as long
+    // as starting the threads saves
+    static constexpr size_t LEAST = (size_t)16 << 20;
+    char* pinned = nullptr;
+    hipEvent_t ev[SLOTS] = {};
+};
 
 struct ProfRec {
     const char* name;
@@ -178,6 +193,8 @@ struct lbm_ctx {
     bool overlap = true;
     int refresh_iters = 0;
     int bcap = 0, lcap = 0;
+
+    Stage stage;
 
     bool prof = false;
     std::vector<ProfRec> pending;
@@ -486,6 +503,9 @@ void release(lbm_ctx* c)
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c->low_count_host) (void)hipHostFree(c->low_count_host);
+    if (c->stage.pinned) (void)hipHostFree(c->stage.pinned);
+    for (hipEvent_t e : c->stage.ev)
+        if (e) (void)hipEventDestroy(e);
     if (c->ev_save) (void)hipEventDestroy(c->ev_save);
     if (c->tstream) {  // an asynchronous refresh may still read the capture rows
         (void)hipStreamSynchronize(c->tstream);
@@ -506,6 +526,127 @@ void release(lbm_ctx* c)
     if (c->net_ready) sur::mlp_free(c->net);
     if (c->work.cap) sur::work_free(c->work);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+}
+
+// Downloads `bytes` of device memory in stream order: put(src, offset, len)
+// receives each chunk in pinned host memory, in any order and from several
+// threads, and copies or converts it to its place.  A copy to pageable memory
+// runs at one thread's pace, which faults in the caller's new pages and copies
+// them; eight threads do both while the bus brings the next chunks.  Five
+// fields of 258^3 values: 73.6 -> 26 ms; nine binary32 planes of 258x130x130,
+// converted on the way: 57.9 -> 5.6 ms.
+// False when nothing was staged (a small copy, or no threads or pinned memory to
+// be had): the caller copies by itself.
+template <typename Put>
+bool staged_download(lbm_ctx* c, const void* dev, size_t bytes, Put put, int* rc)
+{
+    *rc = LBM_OK;
+    Stage& st = c->stage;
+    if (bytes < Stage::LEAST) return false;
+    if (!st.pinned) {
+        bool ok = hipHostMalloc((void**)&st.pinned, Stage::SLOTS * Stage::CHUNK) == hipSuccess;
+        for (hipEvent_t& e : st.ev) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+        if (!ok) {
+            (void)hipGetLastError();
+            if (st.pinned) (void)hipHostFree(st.pinned);
+            st.pinned = nullptr;
+            return false;
+        }
+    }
+    const size_t chunks = (bytes + Stage::CHUNK - 1) / Stage::CHUNK;
+    std::atomic<size_t> queued{0};            // chunks whose copy and event are on the stream
+    std::atomic<int> error{hipSuccess};
+    std::atomic<bool> stop{false};
+    std::atomic<bool> full[Stage::SLOTS];     // the slot holds a chunk not yet put in its place
+    for (auto& f : full) f.store(false);
+    auto work = [&](int w) {
+        (void)hipSetDevice(c->cfg.device);
+        for (size_t k = w; k < chunks; k += Stage::WORKERS) {
+            while (queued.load(std::memory_order_acquire) <= k) {
+                if (stop.load()) return;
+                std::this_thread::yield();
+            }
+            const int slot = (int)(k % Stage::SLOTS);
+            const hipError_t e = hipEventSynchronize(st.ev[slot]);
+            if (e != hipSuccess) {
+                error.store(e);
+                stop.store(true);
+                return;
+            }
+            const size_t off = k * Stage::CHUNK;
+            put(st.pinned + slot * Stage::CHUNK, off, std::min(Stage::CHUNK, bytes - off));
+            full[slot].store(false, std::memory_order_release);
+        }
+    };
+    std::thread pool[Stage::WORKERS];
+    bool started = true;
+    try {
+        for (int w = 0; w < Stage::WORKERS; ++w) pool[w] = std::thread(work, w);
+    } catch (const std::exception&) {  // no thread to be had: nothing is queued yet
+        started = false;
+        stop.store(true);
+    }
+    if (started)
+        for (size_t k = 0; k < chunks && !stop.load(); ++k) {
+            const int slot = (int)(k % Stage::SLOTS);
+            while (full[slot].load(std::memory_order_acquire) && !stop.load()) std::this_thread::yield();
+            if (stop.load()) break;
+            const size_t off = k * Stage::CHUNK;
+            hipError_t e = hipMemcpyAsync(st.pinned + slot * Stage::CHUNK, static_cast<const char*>(dev) + off,
+                                          std::min(Stage::CHUNK, bytes - off), hipMemcpyDeviceToHost, c->stream);
+            if (e == hipSuccess) e = hipEventRecord(st.ev[slot], c->stream);
+            if (e != hipSuccess) {
+                error.store(e);
+                stop.store(true);
+                break;
+            }
+            full[slot].store(true, std::memory_order_release);
+            queued.store(k + 1, std::memory_order_release);
+        }
+    for (auto& t : pool)
+        if (t.joinable()) t.join();
+    if (!started) return false;
+    if (error.load() != hipSuccess) {
+        (void)hipStreamSynchronize(c->stream);  // no copy may still write the slots
+        *rc = fail(c, LBM_E_HIP, std::string("download: ") + hipGetErrorString((hipError_t)error.load()));
+    }
+    return true;
+}
+
+// `count` stored values (binary32 or binary64) of `n`-value planes to doubles;
+// binary32 planes with their shift ref[plane] added where ref is given.
+int download_values(lbm_ctx* c, const void* dev, size_t count, bool f32, size_t n, const double* ref, double* host)
+{
+    int rc;
+    if (!f32) {
+        if (staged_download(c, dev, count * 8, [&](const char* src, size_t off, size_t len) {
+                std::memcpy(reinterpret_cast<char*>(host) + off, src, len);
+            }, &rc))
+            return rc;
+        HIP_TRY(c, hipMemcpyAsync(host, dev, count * 8, hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        return LBM_OK;
+    }
+    auto convert = [&](const float* src, size_t first, size_t m) {
+        for (size_t i = 0; i < m;) {
+            const size_t plane = (first + i) / n, end = std::min(m, (plane + 1) * n - first);
+            if (ref) {
+                const double r = ref[plane];
+                for (; i < end; ++i) host[first + i] = (double)src[i] + r;
+            } else {
+                for (; i < end; ++i) host[first + i] = (double)src[i];
+            }
+        }
+    };
+    if (staged_download(c, dev, count * 4, [&](const char* src, size_t off, size_t len) {
+            convert(reinterpret_cast<const float*>(src), off / 4, len / 4);
+        }, &rc))
+        return rc;
+    std::vector<float> tmp(count);
+    HIP_TRY(c, hipMemcpyAsync(tmp.data(), dev, count * 4, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    convert(tmp.data(), 0, count);
+    return LBM_OK;
 }
 
 int check_field(lbm_ctx* c, int field)
@@ -970,9 +1111,7 @@ int lbm_get_field(lbm_ctx* c, int field, double* host)
     if (int rc = check_field(c, field)) return rc;
     HIP_TRY(c, hipSetDevice(c->cfg.device));
     if (int rc = materialize(c)) return rc;
-    HIP_TRY(c, hipMemcpyAsync(host, c->fld[field], sizeof(double) * c->d.n, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    return LBM_OK;
+    return download_values(c, c->fld[field], c->d.n, false, c->d.n, nullptr, host);
 }
 
 namespace {
@@ -1272,36 +1411,13 @@ int lbm_get_populations(lbm_ctx* c, int which, double* host)
             if (int rc = run_mc(c, McKernel::Unstream, "mc_unstream", 0, 1)) return rc;
         const void* dev = sp ? c->sf[slot] : c->pg[slot];
         const size_t count = (size_t)c->d.n * Q * (sp ? c->ns : 1);
-        if (fp32(c)) {
-            const int64_t n = c->d.n;
-            const double* ref = sp ? c->mfref : c->mgref;
-            std::vector<float> tmp(count);
-            HIP_TRY(c, hipMemcpyAsync(tmp.data(), dev, count * 4, hipMemcpyDeviceToHost, c->stream));
-            HIP_TRY(c, hipStreamSynchronize(c->stream));
-            for (size_t pl = 0; pl < count / n; ++pl)
-                for (int64_t i = 0; i < n; ++i) host[pl * n + i] = (double)tmp[pl * n + i] + ref[pl];
-        } else {
-            HIP_TRY(c, hipMemcpyAsync(host, dev, count * 8, hipMemcpyDeviceToHost, c->stream));
-            HIP_TRY(c, hipStreamSynchronize(c->stream));
-        }
-        return LBM_OK;
+        return download_values(c, dev, count, fp32(c), c->d.n, sp ? c->mfref : c->mgref, host);
     }
     void* buf;
     const double* ref;
     const int slot = pop_slot(c, which, false, &buf, &ref);
     if (slot < 0) return slot;
-    const int64_t n = c->d.n;
-    if (fp32(c)) {
-        std::vector<float> tmp((size_t)n * Q);
-        HIP_TRY(c, hipMemcpyAsync(tmp.data(), buf, tmp.size() * 4, hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-        for (int l = 0; l < Q; ++l)
-            for (int64_t i = 0; i < n; ++i) host[l * n + i] = (double)tmp[l * n + i] + ref[l];
-    } else {
-        HIP_TRY(c, hipMemcpyAsync(host, buf, (size_t)n * Q * 8, hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-    }
-    return LBM_OK;
+    return download_values(c, buf, (size_t)c->d.n * Q, fp32(c), c->d.n, ref, host);
 }
 
 namespace {
@@ -1353,16 +1469,7 @@ int lbm_get_species_field(lbm_ctx* c, int field, double* host)
     size_t cnt;
     if (int rc = species_field_ptr(c, field, &dev, &cnt)) return rc;
     HIP_TRY(c, hipSetDevice(c->cfg.device));
-    if (fp32(c)) {
-        std::vector<float> tmp(cnt);
-        HIP_TRY(c, hipMemcpyAsync(tmp.data(), dev, cnt * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-        std::copy(tmp.begin(), tmp.end(), host);
-    } else {
-        HIP_TRY(c, hipMemcpyAsync(host, dev, cnt * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(c, hipStreamSynchronize(c->stream));
-    }
-    return LBM_OK;
+    return download_values(c, dev, cnt, fp32(c), c->d.n, nullptr, host);
 }
 
 int lbm_init(lbm_ctx* c)
