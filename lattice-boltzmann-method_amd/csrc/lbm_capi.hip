@@ -185,11 +185,12 @@ struct lbm_ctx {
     hipStream_t tstream = nullptr;
     hipEvent_t ev_tstart = nullptr, ev_tdone = nullptr;
     bool refreshing = false;
-    // lbm_step's overlapped schedule: the chemistry on its own stream beside
-    // the transport pass and the mixture collide (LBM_AMD_OVERLAP=0: serial)
+    // lbm_step's overlapped schedule: the chemistry and the mixture energy on
+    // streams of their own beside the species (LBM_AMD_OVERLAP=0: serial)
     int64_t low_max = INT64_MAX;  // LBM_AMD_LOW_MAX: most floor pairs the in-place list may hold at once
-    hipStream_t cstream = nullptr;
-    hipEvent_t ev_cstart = nullptr, ev_cdone = nullptr;
+    hipStream_t cstream = nullptr, estream = nullptr;  // chemistry; mixture energy
+    hipEvent_t ev_cstart = nullptr, ev_cdone = nullptr, ev_trans = nullptr, ev_edone = nullptr;
+    bool energy_streamed = false;  // this step's energy populations are streamed already
     bool overlap = true;
     int refresh_iters = 0;
     int bcap = 0, lcap = 0;
@@ -332,10 +333,14 @@ bool multi(const lbm_ctx* c) { return c->ns > 0; }
 
 bool fp32(const lbm_ctx* c) { return c->cfg.precision == LBM_FP32_SHIFTED; }
 
+int run_mc_on(lbm_ctx* c, hipStream_t s, McKernel k, const char* name, int src, int dst)
+{
+    if (fp32(c)) return launch_on(c, s, name, [&] { launch_mc<float>(k, make_mview<float>(c, src, dst), s); });
+    return launch_on(c, s, name, [&] { launch_mc<double>(k, make_mview<double>(c, src, dst), s); });
+}
 int run_mc(lbm_ctx* c, McKernel k, const char* name, int src, int dst)
 {
-    if (fp32(c)) return launch(c, name, [&] { launch_mc<float>(k, make_mview<float>(c, src, dst), c->stream); });
-    return launch(c, name, [&] { launch_mc<double>(k, make_mview<double>(c, src, dst), c->stream); });
+    return run_mc_on(c, c->stream, k, name, src, dst);
 }
 bool fused(const lbm_ctx* c) { return c->cfg.mode == LBM_MODE_FUSED; }
 
@@ -517,8 +522,12 @@ void release(lbm_ctx* c)
         (void)hipStreamSynchronize(c->cstream);
         (void)hipStreamDestroy(c->cstream);
     }
-    if (c->ev_cstart) (void)hipEventDestroy(c->ev_cstart);
-    if (c->ev_cdone) (void)hipEventDestroy(c->ev_cdone);
+    if (c->estream) {
+        (void)hipStreamSynchronize(c->estream);
+        (void)hipStreamDestroy(c->estream);
+    }
+    for (hipEvent_t e : {c->ev_cstart, c->ev_cdone, c->ev_trans, c->ev_edone})
+        if (e) (void)hipEventDestroy(e);
     if (c->ev_tstart) (void)hipEventDestroy(c->ev_tstart);
     if (c->ev_tdone) (void)hipEventDestroy(c->ev_tdone);
     if (c->tnet.Wf) sur::mlp_free(c->tnet);
@@ -1689,6 +1698,16 @@ int lbm_collide(lbm_ctx* c)
     return LBM_OK;
 }
 
+namespace {
+// The energy populations' stream, unless the step has done it already.
+int stream_energy(lbm_ctx* c)
+{
+    const bool done = c->energy_streamed;
+    c->energy_streamed = false;
+    return done ? LBM_OK : run_mc(c, McKernel::StreamEnergy, "mc_stream_energy", 1, 0);
+}
+}  // namespace
+
 int lbm_stream(lbm_ctx* c)
 {
     if (!c) return LBM_E_ARG;
@@ -1698,14 +1717,14 @@ int lbm_stream(lbm_ctx* c)
             if (!c->pushed)
                 return fail(c, LBM_E_STATE, "lbm_collide_species must run before lbm_stream in the in-place mode");
             c->pushed = false;
-            return run_mc(c, McKernel::StreamEnergy, "mc_stream_energy", 1, 0);
+            return stream_energy(c);
         }
         if (fused(c) && c->push_ready) {  // Collide_Species wrote the streamed species slots of buffer 1
             if (!c->pushed)
                 return fail(c, LBM_E_STATE, "lbm_collide_species must run before lbm_stream in the fused mode");
             std::swap(c->sf[0], c->sf[1]);
             c->pushed = false;
-            return run_mc(c, McKernel::StreamEnergy, "mc_stream_energy", 1, 0);
+            return stream_energy(c);
         }
         if (int rc = run_mc(c, McKernel::Stream, "mc_stream", 1, 0)) return rc;
         if (!fused(c)) return LBM_OK;
@@ -1815,65 +1834,89 @@ int lbm_moments(lbm_ctx* c)
 
 namespace {
 
-// Collide_Species and Collide of one reacting step with the chemistry on a
-// second stream.  The chemistry reads the fields and species
-// planes of the last calculate_moment and writes only its own outputs
-// (sources, heat release, the fallback list, capture rows); the transport
-// pass and the mixture collide neither read nor write those, so the whole
-// chemistry (network pass and fallback list) runs beside them and the push
-// collide, which needs its sources, waits for it.  Each kernel sees exactly
-// the inputs of the serial calls: the state is bitwise that of
-// lbm_collide_species followed by lbm_collide.  (Measured on the 256x128x128
-// layer: 557 against 538 MLUPS serial; the chemistry beside the mixture
-// collide alone, or the fallback list after the wait, gained less.)
+// Collide_Species and Collide of one step (and, where only the energy
+// populations stream, their stream) on three streams:
+//   chemistry   network pass and fallback list, or the plain integrator
+//   energy      the mixture collide, then the energy populations' stream
+//   step        the transport pass, then (with the chemistry's sources) the
+//               species collide
+// The chemistry and the transport pass read the fields and species planes of
+// the last calculate_moment and write only their own outputs; the mixture
+// collide reads the same (on the FP32 path also the transport pass's rates, so
+// it waits for that pass) and writes the energy populations, which nothing else
+// touches; so each kernel sees exactly the inputs of the serial calls and the
+// state is bitwise that of lbm_collide_species followed by lbm_collide and the
+// stream.  Small grids gain most, whose kernels are chains of dependent
+// operations on a few wavefronts.  A step with the chemistry alone beside the
+// rest, and as here: 16x12x10 with two charges 95.5 and 89.7 us, the 2048x4x4
+// flame 505 and 477, the 128x96x48 layer 1925 and 1874.
+// With a network the energy part stays on the step's stream: the network pass
+// is short, and a third kernel beside it stretches it until the chemistry
+// stage takes longer than the integrator's (128x96x64 in FP64: 0.97 of its
+// speed, 1.3 with two streams), for 1 % of the step (256x128x128 in FP32:
+// 6700 us with two streams, 6640 with three).
 int collide_overlapped(lbm_ctx* c)
 {
     HIP_TRY(c, hipSetDevice(c->cfg.device));
-    if (!c->cstream) {
-        HIP_TRY(c, hipStreamCreateWithFlags(&c->cstream, hipStreamNonBlocking));
-        HIP_TRY(c, hipEventCreateWithFlags(&c->ev_cstart, hipEventDisableTiming));
-        HIP_TRY(c, hipEventCreateWithFlags(&c->ev_cdone, hipEventDisableTiming));
+    if (!c->ev_edone) {
+        for (hipStream_t* st : {&c->cstream, &c->estream})
+            if (!*st) HIP_TRY(c, hipStreamCreateWithFlags(st, hipStreamNonBlocking));
+        for (hipEvent_t* e : {&c->ev_cstart, &c->ev_cdone, &c->ev_trans, &c->ev_edone})
+            if (!*e) HIP_TRY(c, hipEventCreateWithFlags(e, hipEventDisableTiming));
     }
     if (inplace(c) && c->pushed)
         return fail(c, LBM_E_STATE,
                     "the in-place mode's species are already collided into the next layout: lbm_stream must "
                     "follow lbm_collide_species");
+    const bool chem = c->cfg.reaction;
+    const bool push = fused(c) && c->push_ready;
     HIP_TRY(c, hipEventRecord(c->ev_cstart, c->stream));
     HIP_TRY(c, hipStreamWaitEvent(c->cstream, c->ev_cstart, 0));
+    const hipStream_t es = c->sur_on ? c->stream : c->estream;
+    if (es != c->stream) HIP_TRY(c, hipStreamWaitEvent(es, c->ev_cstart, 0));
     // the in-place mode's save pass (it reads the species populations and
-    // densities, which the chemistry leaves alone)
-    if (inplace(c))
-        if (int rc = aa_save(c)) {
-            (void)hipEventRecord(c->ev_cdone, c->cstream);
-            return rc;
-        }
-    int rc = DISPATCH(c, [&] {
-        const MultiView<P> v = make_mview<P>(c, 0, 1);
-        if (!c->sur_on)
-            return launch_on(c, c->cstream, "mc_chemistry_plain",
-                             [&] { launch_mc<P>(McKernel::ChemistryBeside, v, c->cstream); });
-        int r = launch_on(c, c->cstream, "mc_chemistry_surrogate", [&] {
-            launch_mc_sur_chemistry<P>(v, c->net, c->chem_list, c->chem_count, c->cstream);
-        });
-        if (!r)
-            r = launch_on(c, c->cstream, "mc_chemistry_fallback",
-                          [&] { launch_mc_chem_list<P>(v, c->chem_list, c->chem_count, c->cstream); });
-        return r;
-    }());
-    // recorded whatever happened, so that the main stream's wait ends
-    HIP_TRY(c, hipEventRecord(c->ev_cdone, c->cstream));
+    // densities, which the other passes leave alone)
+    int rc = inplace(c) ? aa_save(c) : LBM_OK;
+    if (!rc && chem)
+        rc = DISPATCH(c, [&] {
+            const MultiView<P> v = make_mview<P>(c, 0, 1);
+            if (!c->sur_on)
+                return launch_on(c, c->cstream, "mc_chemistry_plain",
+                                 [&] { launch_mc<P>(McKernel::ChemistryBeside, v, c->cstream); });
+            int r = launch_on(c, c->cstream, "mc_chemistry_surrogate", [&] {
+                launch_mc_sur_chemistry<P>(v, c->net, c->chem_list, c->chem_count, c->cstream);
+            });
+            if (!r)
+                r = launch_on(c, c->cstream, "mc_chemistry_fallback",
+                              [&] { launch_mc_chem_list<P>(v, c->chem_list, c->chem_count, c->cstream); });
+            return r;
+        }());
+    // (the joins are recorded whatever happened, so that the step's waits end)
+    const hipError_t ec = hipEventRecord(c->ev_cdone, c->cstream);
     if (!rc) rc = run_mc(c, McKernel::SpeciesTransport, "mc_species_transport", 0, 1);
     c->omix_fresh = !rc && fp32(c);
-    if (!rc) rc = run_mc(c, McKernel::Collide, "mc_collide_mixture", 0, 1);
+    hipError_t ee = hipSuccess;
+    if (c->omix_fresh && es != c->stream) {
+        ee = hipEventRecord(c->ev_trans, c->stream);
+        if (ee == hipSuccess) ee = hipStreamWaitEvent(es, c->ev_trans, 0);
+    }
+    if (!rc) rc = run_mc_on(c, es, McKernel::Collide, "mc_collide_mixture", 0, 1);
+    const bool energy = !rc && (push || inplace(c));
+    if (energy) rc = run_mc_on(c, es, McKernel::StreamEnergy, "mc_stream_energy", 1, 0);
+    if (ee == hipSuccess && es != c->stream) ee = hipEventRecord(c->ev_edone, es);
+    HIP_TRY(c, ec);
     HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_cdone, 0));
     if (!rc && inplace(c)) {
         rc = aa_collide_species(c);
-    } else if (!rc && fused(c) && c->push_ready) {
+    } else if (!rc && push) {
         rc = run_mc(c, McKernel::CollideSpeciesPush, "mc_collide_species_push", 0, 1);
         if (!rc) c->pushed = true;
     } else if (!rc) {
         rc = run_mc(c, McKernel::CollideSpecies, "mc_collide_species", 0, 1);
     }
+    HIP_TRY(c, ee);
+    if (es != c->stream) HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_edone, 0));
+    c->energy_streamed = energy && !rc;
     ++c->step;
     return rc;
 }
@@ -1885,8 +1928,8 @@ int lbm_step(lbm_ctx* c, int nsteps)
     if (!c) return LBM_E_ARG;
     for (int s = 0; s < nsteps; ++s) {
         int rc;
-        // every multicomponent step with chemistry takes the overlapped schedule
-        const bool ov = c->overlap && multi(c) && c->types_set && c->cfg.reaction;
+        // every multicomponent step takes the overlapped schedule
+        const bool ov = c->overlap && multi(c) && c->types_set;
         if (ov) {
             if ((rc = collide_overlapped(c))) return rc;
         } else if ((rc = lbm_collide_species(c)) || (rc = lbm_collide(c))) {
