@@ -85,14 +85,13 @@ struct lbm_ctx {
     void* sf[2] = {nullptr, nullptr};
     void* sp_block = nullptr;  // X, rho_a [NS][n] and u_a [3][NS][n], element type of the populations
     chem::Units units{};
-    // TMS_BC outflow interface cells (cell, direction) and unsupported boundary kinds
+    // TMS_BC interface cells (cell, direction): tms_count of the outflow, then
+    // tin_count of the inflow (TYPE_I, TYPE_I_C); unsupported boundary kinds
     int* tms_cell = nullptr;
     int* tms_dir = nullptr;
-    int tms_count = 0;
-    double* tms_rec = nullptr;  // per-cell values between the outflow sweep's launches
-    int* tin_cell = nullptr;  // TMS_BC inflow interface cells (TYPE_I, TYPE_I_C)
-    int* tin_dir = nullptr;
-    int tin_count = 0;
+    int tms_count = 0, tin_count = 0;
+    bool tms_apart = true;      // no cell of one sweep near one of the other
+    double* tms_rec = nullptr;  // per-cell values between the sweeps' launches
     int* twall_cell = nullptr;  // TMS_BC isothermal-wall interface cells (TYPE_S)
     int twall_count = 0;
     std::string tms_unsupported;
@@ -502,7 +501,7 @@ void release(lbm_ctx* c)
                     c->sf[1],     c->sp_block,  c->tms_cell,   c->tms_dir,   c->src,       c->sur_stats,
                     c->stats_part, c->sur_count, c->chem_list, c->chem_count, c->tchem,    c->cap_buf,
                     c->cap_count, c->bx,        c->bt,         c->bloss,     c->mref_dev,  c->sums_part, c->adam_c12, c->train_it,
-                    c->tin_cell,  c->tin_dir,   c->sbc_cell,  c->tsp,        c->omix,       c->twall_cell, c->cjc_cell,
+                    c->sbc_cell,  c->tsp,        c->omix,       c->twall_cell, c->cjc_cell,
                     c->side_slot, c->side_cell, c->fside, c->aa_pending, c->low_cell, c->low_sp,
                     c->low_keep,  c->low_count, c->smooth_tmp, c->tms_rec};
     for (void* p : ptrs)
@@ -1027,22 +1026,32 @@ int lbm_set_types(lbm_ctx* c, const uint8_t* types)
         c->tms_cell = c->tms_dir = nullptr;
         c->tms_rec = nullptr;
         c->tms_count = (int)tcell.size();
-        if (c->tms_count) {
+        c->tin_count = (int)icell.size();
+        // A sweep's targets read and (TYPE_O, TYPE_I) write fields up to two cells
+        // off their entries and follow the other sweep's results there: the two
+        // run at once only with five cells between their entries.
+        constexpr int FAR = 5;
+        c->tms_apart = true;
+        std::vector<uint8_t> near(tcell.empty() || icell.empty() ? 0 : (size_t)d.n, 0);
+        if (!near.empty()) {
+            for (int t : tcell) near[t] = 1;
+            for (int t : icell) {
+                const int i = t / (d.ny * d.nz), j = t / d.nz % d.ny, k = t % d.nz;
+                for (int a = std::max(i - FAR, 0); a <= std::min(i + FAR, d.nx - 1); ++a)
+                    for (int b = std::max(j - FAR, 0); b <= std::min(j + FAR, d.ny - 1); ++b)
+                        for (int e = std::max(k - FAR, 0); e <= std::min(k + FAR, d.nz - 1); ++e)
+                            if (near[((int64_t)a * d.ny + b) * d.nz + e]) c->tms_apart = false;
+                if (!c->tms_apart) break;
+            }
+        }
+        tcell.insert(tcell.end(), icell.begin(), icell.end());
+        tdir.insert(tdir.end(), idir.begin(), idir.end());
+        if (!tcell.empty()) {
             HIP_TRY(c, hipMalloc((void**)&c->tms_cell, sizeof(int) * tcell.size()));
             HIP_TRY(c, hipMalloc((void**)&c->tms_dir, sizeof(int) * tdir.size()));
             HIP_TRY(c, hipMalloc((void**)&c->tms_rec, sizeof(double) * mc_tms_record_fields() * tcell.size()));
             HIP_TRY(c, hipMemcpy(c->tms_cell, tcell.data(), sizeof(int) * tcell.size(), hipMemcpyHostToDevice));
             HIP_TRY(c, hipMemcpy(c->tms_dir, tdir.data(), sizeof(int) * tdir.size(), hipMemcpyHostToDevice));
-        }
-        if (c->tin_cell) (void)hipFree(c->tin_cell);
-        if (c->tin_dir) (void)hipFree(c->tin_dir);
-        c->tin_cell = c->tin_dir = nullptr;
-        c->tin_count = (int)icell.size();
-        if (c->tin_count) {
-            HIP_TRY(c, hipMalloc((void**)&c->tin_cell, sizeof(int) * icell.size()));
-            HIP_TRY(c, hipMalloc((void**)&c->tin_dir, sizeof(int) * idir.size()));
-            HIP_TRY(c, hipMemcpy(c->tin_cell, icell.data(), sizeof(int) * icell.size(), hipMemcpyHostToDevice));
-            HIP_TRY(c, hipMemcpy(c->tin_dir, idir.data(), sizeof(int) * idir.size(), hipMemcpyHostToDevice));
         }
         if (c->twall_cell) (void)hipFree(c->twall_cell);
         c->twall_cell = nullptr;
@@ -1744,15 +1753,22 @@ int lbm_tms_bc(lbm_ctx* c)
         if (!c->types_set) return fail(c, LBM_E_STATE, "lbm_set_types must precede stepping");
         if (!c->tms_unsupported.empty()) return fail(c, LBM_E_UNSUPPORTED, c->tms_unsupported);
         // outflow, inflow and isothermal-wall sweeps (lbm-bc.cpp:126, 463, 941)
-        if (int rc = DISPATCH(c, launch(c, "mc_tms_outflow", [&] {
-                launch_mc_tms<P>(make_mview<P>(c, 0, 0), c->tms_cell, c->tms_dir, c->tms_count, c->tms_rec,
-                                 c->stream);
-            })))
-            return rc;
-        if (int rc = DISPATCH(c, launch(c, "mc_tms_inflow", [&] {
-                launch_mc_tms_in<P>(make_mview<P>(c, 0, 0), c->tin_cell, c->tin_dir, c->tin_count, c->stream);
-            })))
-            return rc;
+        const int out = c->tms_count, in = c->tin_count;
+        // (one set of launches where both sweeps have cells and lie apart)
+        const bool both = out > 0 && in > 0 && c->tms_apart;
+        if (out > 0)
+            if (int rc = DISPATCH(c, launch(c, "mc_tms_outflow", [&] {
+                    launch_mc_tms<P>(make_mview<P>(c, 0, 0), c->tms_cell, c->tms_dir, out, both ? in : 0, c->tms_rec,
+                                     c->stream);
+                })))
+                return rc;
+        if (in > 0 && !both)
+            if (int rc = DISPATCH(c, launch(c, "mc_tms_inflow", [&] {
+                    launch_mc_tms<P>(make_mview<P>(c, 0, 0), c->tms_cell + out, c->tms_dir + out, 0, in, c->tms_rec,
+                                     c->stream);
+                })))
+                return rc;
+        if (c->twall_count <= 0) return LBM_OK;
         return DISPATCH(c, launch(c, "mc_tms_wall", [&] {
             launch_mc_tms_wall<P>(make_mview<P>(c, 0, 0), c->twall_cell, c->twall_count, c->stream);
         }));

@@ -121,17 +121,15 @@ void launch_mc_diag_mach(const MultiView<P>& v, double* partials, hipStream_t s)
 // NSCBC sigma of the partially non-reflecting outflow (NSCBC_SIGMA_OUT, defines.hpp:100-102)
 constexpr double NSCBC_SIGMA_OUT = 0.25;
 
-// TMS_BC outflow reconstruction over `count` interface cells (cell index and
-// the axis-aligned direction whose upstream neighbour is the TYPE_O_C ghost);
-// `rec` holds mc_tms_record_fields() x count doubles of per-cell values.
+// TMS_BC outflow and inflow reconstruction over n_out + n_in interface cells, the
+// outflow's first (cell index and the axis-aligned direction whose upstream
+// neighbour is the ghost); `rec` holds mc_tms_record_fields() doubles of each.
+// The sweeps run at once: a cell of one must not be near a cell of the other.
 template <typename P>
-void launch_mc_tms(const MultiView<P>& v, const int* cells, const int* dirs, int count, double* rec, hipStream_t s);
+void launch_mc_tms(const MultiView<P>& v, const int* cells, const int* dirs, int n_out, int n_in, double* rec,
+                   hipStream_t s);
 int mc_tms_record_fields();
 
-// TMS_BC inflow reconstruction for TYPE_I_C ghosts (same list layout; runs
-// after the outflow sweep).
-template <typename P>
-void launch_mc_tms_in(const MultiView<P>& v, const int* cells, const int* dirs, int count, hipStream_t s);
 // TMS_BC isothermal-wall sweep (TYPE_S) on the interface cells `cells`
 template <typename P>
 void launch_mc_tms_wall(const MultiView<P>& v, const int* cells, int count, hipStream_t s);

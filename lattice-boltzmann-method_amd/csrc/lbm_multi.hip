@@ -1922,31 +1922,60 @@ __device__ inline void sound_DP(const Units& u, double rho, double p, const doub
 
 }  // namespace
 
-// The sweep runs in four launches over a record of per-entry values
-// (tms_rec, [TR_*][count] doubles), one thread per entry or per (entry,
-// population set), with the arithmetic of a single per-cell pass:
-//   k_mc_tms_target   the target state (TYPE_O: calculate_moment_point of the
-//                     downstream cell; TYPE_O_C: the NSCBC LODI step);
-//   k_mc_tms_local    per (entry, species): the local moments with the target
-//                     populations in the unknown directions;
-//   k_mc_tms_close    per entry: mixture sums, calculate_temp, local state;
-//   k_mc_tms_rebuild  per (entry, species or energy): the reconstruction.
-// Each entry is a distinct cell, and only the last launch writes populations,
-// each thread those of its own cell.
+// The outflow and inflow sweeps run in two launches over a list of entries,
+// the outflow's before the inflow's, and a record of per-entry values (tms_rec,
+// [TR_*][count] doubles):
+//   k_mc_tms_target   one thread per entry: the target state;
+//   k_mc_tms_sweep    the local moments with the target populations in the
+//                     unknown directions, calculate_temp and the local state,
+//                     and the reconstruction: 2 (outflow) f_tgt - f_loc.
+// Each entry is a distinct cell, a target reads populations of none but cells
+// downstream of its entry, and only the second launch writes populations, each
+// thread those of its own cell.
 enum {
-    TR_RHO_OUT = 0, TR_VOUT = 1, TR_TSO = 4, TR_U_OUT = 5, TR_TH_OUT = 6, TR_MASK = 7, TR_RA_OUT = 8,
-    TR_RA_LOC = TR_RA_OUT + NS, TR_MA = TR_RA_LOC + NS, TR_RHO_LOC = TR_MA + 3 * NS, TR_VLOC = TR_RHO_LOC + 1,
-    TR_TSL = TR_VLOC + 3, TR_U_LOC = TR_TSL + 1, TR_TH_LOC = TR_U_LOC + 1, TR_COUNT = TR_TH_LOC + 1
+    TR_RHO = 0, TR_V = 1, TR_TS = 4, TR_U = 5, TR_TH = 6, TR_MASK = 7, TR_RA = 8, TR_COUNT = TR_RA + NS
 };
 
+// The record of entry t of `count`; Y is normalised, Ts the target's SI
+// temperature, ghosts the two cell types whose populations are unknown.
 template <typename P>
-__global__ __launch_bounds__(64) void k_mc_tms_target(MultiView<P> v, const int* cells, const int* dirs, int count,
-                                                      double* rec)
+__device__ inline void tms_record(const MultiView<P>& v, int c, int t, int count, double* rec, double rho,
+                                  const double vel[3], double Ts, const double ra[NS], const double Y[NS], uint8_t g0,
+                                  uint8_t g1)
 {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= count) return;
-    const int c = cells[t], l = dirs[t];
     const Ijk x = ijk(v.d, c);
+    uint32_t unknown = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const uint8_t tq = v.type[cell(v.d, x.i - cx(q), x.j - cy(q), x.k - cz(q))];
+        if (tq == g0 || tq == g1) unknown |= 1u << q;
+    }
+    auto R = [&](int f) -> double& { return rec[(int64_t)f * count + t]; };
+    R(TR_RHO) = rho;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) R(TR_V + d) = vel[d];
+    R(TR_TS) = Ts;
+    // equilibria of the target state (calculate_feq_geq, lbm-edf.cpp:198-209)
+    R(TR_U) = v.u.energy_mass(u_mass(Ts, Y));
+    R(TR_TH) = v.u.energy_mass(R_UNIV * Ts / mean_W(Y));
+    R(TR_MASK) = (double)unknown;
+#pragma unroll
+    for (int a = 0; a < NS; ++a) R(TR_RA + a) = ra[a];
+}
+
+// x[i] of three values, and x[i] = r: an array indexed by a variable would live
+// in scratch memory, each use a load on the target's chain
+__device__ inline double pick(const double* x, int i) { return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]); }
+__device__ inline void put(double* x, int i, double r)
+{
+#pragma unroll
+    for (int d = 0; d < 3; ++d) x[d] = d == i ? r : x[d];
+}
+
+// The outflow target: TYPE_O the moments downstream, TYPE_O_C the NSCBC LODI step.
+template <typename P>
+__device__ inline void tms_outflow_target(const MultiView<P>& v, int c, int l, int t, int count, double* rec)
+{
     const int strides[3] = {v.d.ny * v.d.nz, v.d.nz, 1};
     const int Ns[3] = {v.d.nx - 2, v.d.ny - 2, v.d.nz - 2};
     const int dims[3] = {v.d.nx, v.d.ny, v.d.nz};
@@ -2011,13 +2040,13 @@ __global__ __launch_bounds__(64) void k_mc_tms_target(MultiView<P> v, const int*
         }
         if (any) {
             // Yoo & Im transverse terms for the normal direction idir
-            T1 = vel[t1] * (Dt[0][0] - rho * a_s * Dt[0][1 + idir]) + vel[t2] * (Dt[1][0] - rho * a_s * Dt[1][1 + idir]) +
-                 gam * p * (Dt[0][1 + t1] + Dt[1][1 + t2]);
-            T5 = vel[t1] * (Dt[0][0] + rho * a_s * Dt[0][1 + idir]) + vel[t2] * (Dt[1][0] + rho * a_s * Dt[1][1 + idir]) +
-                 gam * p * (Dt[0][1 + t1] + Dt[1][1 + t2]);
+            T1 = pick(vel, t1) * (Dt[0][0] - rho * a_s * pick(Dt[0] + 1, idir)) + pick(vel, t2) * (Dt[1][0] - rho * a_s * pick(Dt[1] + 1, idir)) +
+                 gam * p * (pick(Dt[0] + 1, t1) + pick(Dt[1] + 1, t2));
+            T5 = pick(vel, t1) * (Dt[0][0] + rho * a_s * pick(Dt[0] + 1, idir)) + pick(vel, t2) * (Dt[1][0] + rho * a_s * pick(Dt[1] + 1, idir)) +
+                 gam * p * (pick(Dt[0] + 1, t1) + pick(Dt[1] + 1, t2));
         }
     }
-    const double un = vel[idir], dun = Dn[1 + idir], dpn = Dn[0], drhon = Dn[4];
+    const double un = pick(vel, idir), dun = pick(Dn + 1, idir), dpn = Dn[0], drhon = Dn[4];
     const double mach = sqrt(vel[0] * vel[0] + vel[1] * vel[1] + vel[2] * vel[2]) / a_s;
     double L1 = (un - a_s) * (dpn - rho * a_s * dun);
     double L5 = (un + a_s) * (dpn + rho * a_s * dun);
@@ -2042,155 +2071,7 @@ __global__ __launch_bounds__(64) void k_mc_tms_target(MultiView<P> v, const int*
     double Tsi_out;
     T_out = T_from_DP(v.u, rho_out, p_out, Yo, &Tsi_out);
     }
-    // ---- equilibria of the target state (calculate_feq_geq, lbm-edf.cpp:198-209)
-    const double Tso = v.u.si_temp(T_out);
-    uint32_t unknown = 0;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const uint8_t tq = v.type[cell(v.d, x.i - cx(q), x.j - cy(q), x.k - cz(q))];
-        if (tq == TYPE_O || tq == TYPE_O_C) unknown |= 1u << q;
-    }
-    auto R = [&](int f) -> double& { return rec[(int64_t)f * count + t]; };
-    R(TR_RHO_OUT) = rho_out;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) R(TR_VOUT + d) = vout[d];
-    R(TR_TSO) = Tso;
-    R(TR_U_OUT) = v.u.energy_mass(u_mass(Tso, Yo));
-    R(TR_TH_OUT) = v.u.energy_mass(R_UNIV * Tso / mean_W(Yo));
-    R(TR_MASK) = (double)unknown;
-#pragma unroll
-    for (int a = 0; a < NS; ++a) R(TR_RA_OUT + a) = ra_out[a];
-}
-
-// grid (count / 64, NS): local moments of species blockIdx.y
-template <typename P>
-__global__ __launch_bounds__(64) void k_mc_tms_local(MultiView<P> v, const int* cells, int count, double* rec)
-{
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= count) return;
-    const int a = blockIdx.y;
-    const int c = cells[t];
-    auto R = [&](int f) -> double& { return rec[(int64_t)f * count + t]; };
-    const uint32_t unknown = (uint32_t)R(TR_MASK);
-    const double vout[3] = {R(TR_VOUT), R(TR_VOUT + 1), R(TR_VOUT + 2)};
-    const double ra_out = R(TR_RA_OUT + a);
-    const double zero[3] = {0, 0, 0};
-    const double th_a = v.u.energy_mass(R_UNIV * R(TR_TSO) / W[a]);
-    Axis3<double> Fo[3];
-    feq_axes<double>(Fo, vout, th_a, zero);
-    double r = 0, m0 = 0, m1 = 0, m2 = 0;
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const double f = (unknown >> q & 1u) ? feq_dir<double>(Fo, q, ra_out) : ldf_in(v, a, q, c);
-        r += f;
-        if (cx(q)) m0 += cx(q) * f;
-        if (cy(q)) m1 += cy(q) * f;
-        if (cz(q)) m2 += cz(q) * f;
-    }
-    R(TR_RA_LOC + a) = r;
-    R(TR_MA + 3 * a) = m0;
-    R(TR_MA + 3 * a + 1) = m1;
-    R(TR_MA + 3 * a + 2) = m2;
-}
-
-template <typename P>
-__global__ __launch_bounds__(64) void k_mc_tms_close(MultiView<P> v, const int* cells, int count, double* rec)
-{
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= count) return;
-    const int c = cells[t];
-    double* const* Fd = v.fld;
-    auto R = [&](int f) -> double& { return rec[(int64_t)f * count + t]; };
-    const uint32_t unknown = (uint32_t)R(TR_MASK);
-    const double rho_out = R(TR_RHO_OUT), th_out = R(TR_TH_OUT), U_out = R(TR_U_OUT);
-    const double vout[3] = {R(TR_VOUT), R(TR_VOUT + 1), R(TR_VOUT + 2)};
-    double re_loc = 0, rho_loc = 0, mloc[3] = {0, 0, 0};
-    const GeqAxes<double> Go = geq_axes<double>(th_out, vout);
-#pragma unroll
-    for (int q = 0; q < Q; ++q)
-        re_loc += (unknown >> q & 1u) ? geq_dir<double>(Go, q, rho_out, U_out - 1.5 * th_out)
-                                      : ldg(v, v.g, q, c);
-    double ra_loc[NS], ma[NS][3];
-    for (int a = 0; a < NS; ++a) {
-        ra_loc[a] = R(TR_RA_LOC + a);
-        rho_loc += ra_loc[a];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            ma[a][d] = R(TR_MA + 3 * a + d);
-            mloc[d] += ma[a][d];
-            ma[a][d] = ra_loc[a] > 0.0 ? ma[a][d] / ra_loc[a] : 0.0;
-            R(TR_MA + 3 * a + d) = ma[a][d];
-        }
-    }
-    double vloc[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) vloc[d] = rho_loc > 0 ? mloc[d] / rho_loc : 0.0;
-    double Uloc = re_loc / rho_loc;
-    for (int a = 0; a < NS; ++a)
-        Uloc = Uloc - 0.5 * ra_loc[a] / rho_loc * (ma[a][0] * ma[a][0] + ma[a][1] * ma[a][1] + ma[a][2] * ma[a][2]);
-    // calculate_temp (lbm-moment.cpp:540-553)
-    double Yl[NS];
-#pragma unroll
-    for (int a = 0; a < NS; ++a) Yl[a] = ra_loc[a] / rho_loc;
-    normalize(Yl);
-    const double T_loc = v.u.temp(T_from_UV(v.u.si_energy_mass(Uloc), Yl, v.u.si_temp(Fd[LBM_FIELD_T][c])));
-    const double Tsl = v.u.si_temp(T_loc);
-    R(TR_RHO_LOC) = rho_loc;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) R(TR_VLOC + d) = vloc[d];
-    R(TR_TSL) = Tsl;
-    R(TR_U_LOC) = v.u.energy_mass(u_mass(Tsl, Yl));
-    R(TR_TH_LOC) = v.u.energy_mass(R_UNIV * Tsl / mean_W(Yl));
-}
-
-// grid (count / 64, NS + 1): reconstruction of species blockIdx.y (NS: the
-// energy populations); unknown 2 f_out - f_loc, known f_out + f - f_loc
-template <typename P>
-__global__ __launch_bounds__(64) void k_mc_tms_rebuild(MultiView<P> v, const int* cells, int count, const double* rec)
-{
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= count) return;
-    const int a = blockIdx.y;
-    const int c = cells[t];
-    auto R = [&](int f) { return rec[(int64_t)f * count + t]; };
-    const uint32_t unknown = (uint32_t)R(TR_MASK);
-    const double vout[3] = {R(TR_VOUT), R(TR_VOUT + 1), R(TR_VOUT + 2)};
-    if (a < NS) {
-        const double zero[3] = {0, 0, 0};
-        const double ma[3] = {R(TR_MA + 3 * a), R(TR_MA + 3 * a + 1), R(TR_MA + 3 * a + 2)};
-        const double ra_out = R(TR_RA_OUT + a), ra_loc = R(TR_RA_LOC + a);
-        const double tho = v.u.energy_mass(R_UNIV * R(TR_TSO) / W[a]);
-        const double thl = v.u.energy_mass(R_UNIV * R(TR_TSL) / W[a]);
-        Axis3<double> Fo[3], Fl[3];
-        feq_axes<double>(Fo, vout, tho, zero);
-        feq_axes<double>(Fl, ma, thl, zero);
-        // every load before the first store: the stores go to the same
-        // population set, so interleaved they would serialise the loads
-        double fin[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) fin[q] = ldf_in(v, a, q, c);
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const double fo = feq_dir<double>(Fo, q, ra_out);
-            const double flc = feq_dir<double>(Fl, q, ra_loc);
-            stf_in(v, a, q, c, (unknown >> q & 1u) ? 2 * fo - flc : fo + fin[q] - flc);
-        }
-        return;
-    }
-    const double rho_out = R(TR_RHO_OUT), th_out = R(TR_TH_OUT), U_out = R(TR_U_OUT);
-    const double rho_loc = R(TR_RHO_LOC), th_loc = R(TR_TH_LOC), U_loc = R(TR_U_LOC);
-    const double vloc[3] = {R(TR_VLOC), R(TR_VLOC + 1), R(TR_VLOC + 2)};
-    const GeqAxes<double> Go = geq_axes<double>(th_out, vout);
-    const GeqAxes<double> Gl = geq_axes<double>(th_loc, vloc);
-    double gin[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) gin[q] = ldg(v, v.g, q, c);
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const double go = geq_dir<double>(Go, q, rho_out, U_out - 1.5 * th_out);
-        const double gl = geq_dir<double>(Gl, q, rho_loc, U_loc - 1.5 * th_loc);
-        stg(v, v.g, q, c, (unknown >> q & 1u) ? 2 * go - gl : go + gin[q] - gl);
-    }
+    tms_record(v, c, t, count, rec, rho_out, vout, v.u.si_temp(T_out), ra_out, Yo, TYPE_O, TYPE_O_C);
 }
 
 // ------------------------------------------------- TMS_BC inflow sweep
@@ -2203,13 +2084,9 @@ __global__ __launch_bounds__(64) void k_mc_tms_rebuild(MultiView<P> v, const int
 // (inflow populations substituted) and f_tgt that of the local density and
 // composition at the inflow velocity and temperature.
 template <typename P>
-__global__ __launch_bounds__(64) void k_mc_tms_in(MultiView<P> v, const int* cells, const int* dirs, int count)
+__device__ inline void tms_inflow_target(const MultiView<P>& v, int c, int l, int t, int count, double* rec)
 {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= count) return;
-    const int c = cells[t], l = dirs[t];
     const int64_t n = v.d.n;
-    const Ijk x = ijk(v.d, c);
     const int strides[3] = {v.d.ny * v.d.nz, v.d.nz, 1};
     const int dims[3] = {v.d.nx, v.d.ny, v.d.nz};
     const int cl[3] = {cx(l), cy(l), cz(l)};
@@ -2256,7 +2133,7 @@ __global__ __launch_bounds__(64) void k_mc_tms_in(MultiView<P> v, const int* cel
     const double du = fd_uw(Fd[LBM_FIELD_U + idir][c], Fd[LBM_FIELD_U + idir][c1]);
     const double dp = fd_uw(p, Fd[LBM_FIELD_P][c1]);
     const double rho1 = Fd[LBM_FIELD_RHO][c1];
-    const double un = vel[idir];
+    const double un = pick(vel, idir);
     // tangential components as paired per normal: x -> (v, w), y -> (w, u), z -> (u, v)
     const int t3 = idir == 0 ? 1 : (idir == 1 ? 2 : 0);
     const int t4 = idir == 0 ? 2 : (idir == 1 ? 0 : 1);
@@ -2264,23 +2141,23 @@ __global__ __launch_bounds__(64) void k_mc_tms_in(MultiView<P> v, const int* cel
     const double Rmix = v.u.cp(R_UNIV / mean_W(Yn));
     double L1 = (un - a_s) * (dp - rho * a_s * du);
     const double L2 = sigma * a_s / Nd * rho * Rmix * (Fd[LBM_FIELD_T][c] - Fd[LBM_FIELD_T][cb]);
-    const double L3 = sigma * a_s / Nd * (vel[t3] - velb[t3]);
-    const double L4 = sigma * a_s / Nd * (vel[t4] - velb[t4]);
+    const double L3 = sigma * a_s / Nd * (pick(vel, t3) - pick(velb, t3));
+    const double L4 = sigma * a_s / Nd * (pick(vel, t4) - pick(velb, t4));
     double L5 = (un + a_s) * (dp + rho * a_s * du);
     const double K = sigma * a_s * a_s / Nd * rho * (1.0 - (un / a_s) * (un / a_s));
     // the z-normal branch tests cy (lbm-bc.cpp:652), so it always takes the second form
     const bool left = idir == 2 ? (cy(l) > 0) : (isign > 0);
-    if (left) L5 = K * (un - velb[idir]);
-    else L1 = K * (un - velb[idir]);
+    if (left) L5 = K * (un - pick(velb, idir));
+    else L1 = K * (un - pick(velb, idir));
     const double d1 = 1.0 / (a_s * a_s) * (L2 + 0.5 * (L5 + L1));
     const double d2 = 1.0 / (2.0 * rho * a_s) * (L5 - L1);
     const double d5 = 0.5 * (L5 + L1);
     rho_in = rho - 1 * d1;
 #pragma unroll
     for (int d = 0; d < 3; ++d) vin[d] = vel[d];
-    vin[idir] = vel[idir] - 1 * d2;
-    vin[t3] = vel[t3] - 1 * L3;
-    vin[t4] = vel[t4] - 1 * L4;
+    put(vin, idir, pick(vel, idir) - 1 * d2);
+    put(vin, t3, pick(vel, t3) - 1 * L3);
+    put(vin, t4, pick(vel, t4) - 1 * L4);
     p_in = p - 1 * d5;
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
@@ -2296,92 +2173,161 @@ __global__ __launch_bounds__(64) void k_mc_tms_in(MultiView<P> v, const int* cel
     rho_in = v.u.rho(v.u.si_p(p_in) * mean_W(Yi) / (R_UNIV * Tsi));
 #pragma unroll
     for (int a = 0; a < NS; ++a) ra_in[a] = Yi[a] * rho_in;
-    // ---- equilibria of the inflow state (calculate_feq_geq, lbm-edf.cpp:198-209)
-    const double U_in = v.u.energy_mass(u_mass(Tsi, Yi));
-    const double th_in = v.u.energy_mass(R_UNIV * Tsi / mean_W(Yi));
+    tms_record(v, c, t, count, rec, rho_in, vin, Tsi, ra_in, Yi, TYPE_I, TYPE_I_C);
+}
+
+// Entries [0, n_out) are the outflow's, the other n_in the inflow's; each kind
+// in blocks of its own.
+template <typename P>
+__global__ __launch_bounds__(64) void k_mc_tms_target(MultiView<P> v, const int* cells, const int* dirs, int n_out,
+                                                      int n_in, double* rec)
+{
+    const int nb_out = (n_out + 63) / 64;
+    if ((int)blockIdx.x < nb_out) {
+        const int t = blockIdx.x * 64 + threadIdx.x;
+        if (t < n_out) tms_outflow_target(v, cells[t], dirs[t], t, n_out + n_in, rec);
+    } else {
+        const int t = n_out + ((int)blockIdx.x - nb_out) * 64 + threadIdx.x;
+        if (t < n_out + n_in) tms_inflow_target(v, cells[t], dirs[t], t, n_out + n_in, rec);
+    }
+}
+
+// The rest of both sweeps, a block for TMS_E entries: one thread per (entry,
+// species) and one wavefront for the entries' energy populations and mixture
+// sums.  A sweep is a chain of dependent operations on a few interface cells
+// (the 2048x4x4 flame: 16 at each end), so what counts is how long one thread's
+// part of it is.  The outflow's rest in three launches and the inflow in one
+// thread per cell took 49 and 125 us of that flame's step; with both sweeps
+// here 40 steps of it went from 20.4 to 13.8 ms (128x96x48 layer, 12288
+// outflow cells: 68.1 to 67.5 ms of 30 steps).
+constexpr int TMS_E = NS <= 16 ? 16 : 8;  // TMS_E NS <= 512: 128 registers and more
+constexpr int TMS_ROW = (TMS_E * NS + 63) / 64 * 64;
+template <typename P>
+__global__ __launch_bounds__(TMS_ROW + 64) void k_mc_tms_sweep(MultiView<P> v, const int* cells, int n_out, int count,
+                                                               const double* rec)
+{
+    enum { RA = 0, M = NS, S = 4 * NS, TSL = 5 * NS, FIELDS };
+    __shared__ double sh[FIELDS][TMS_E];
+    const bool energy = threadIdx.x >= TMS_ROW;
+    const int e = threadIdx.x % TMS_E, a = energy ? NS : threadIdx.x / TMS_E;
+    const int t = blockIdx.x * TMS_E + e;
+    const bool on = t < count && (energy ? threadIdx.x - TMS_ROW < TMS_E : a < NS);
+    const int c = on ? cells[t] : 0;
+    const bool inflow = t >= n_out;
+    auto R = [&](int f) { return rec[(int64_t)f * count + t]; };
     uint32_t unknown = 0;
+    double vt[3], rho_t, th_t, U_t = 0, ra_loc = 0, m[3], fin[Q];
+    if (on) {
+        unknown = (uint32_t)R(TR_MASK);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const uint8_t tq = v.type[cell(v.d, x.i - cx(q), x.j - cy(q), x.k - cz(q))];
-        if (tq == TYPE_I || tq == TYPE_I_C) unknown |= 1u << q;
+        for (int d = 0; d < 3; ++d) vt[d] = R(TR_V + d);
     }
     const double zero[3] = {0, 0, 0};
-    // ---- local moments with the inflow populations in the unknown directions
-    double ra_loc[NS], ma[NS][3], re_loc = 0;
-    double rho_loc = 0, mloc[3] = {0, 0, 0};
-    for (int a = 0; a < NS; ++a) {
-        const double th_a = v.u.energy_mass(R_UNIV * Tsi / W[a]);
-        Axis3<double> Fi[3];
-        feq_axes<double>(Fi, vin, th_a, zero);
-        double r = 0, m0 = 0, m1 = 0, m2 = 0;
+    // ---- local moments with the target populations in the unknown directions
+    // (all loads stand before the first store: the stores go to the same
+    // population set, so interleaved they would serialise the loads)
+    if (on && !energy) {
+        rho_t = R(TR_RA + a);
+        th_t = v.u.energy_mass(R_UNIV * R(TR_TS) / W[a]);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) fin[q] = ldf_in(v, a, q, c);
+        Axis3<double> Ft[3];
+        feq_axes<double>(Ft, vt, th_t, zero);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) m[d] = 0;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const double f = (unknown >> q & 1u) ? feq_dir<double>(Fi, q, ra_in[a]) : ldf_in(v, a, q, c);
-            r += f;
-            if (cx(q)) m0 += cx(q) * f;
-            if (cy(q)) m1 += cy(q) * f;
-            if (cz(q)) m2 += cz(q) * f;
+            const double f = (unknown >> q & 1u) ? feq_dir<double>(Ft, q, rho_t) : fin[q];
+            ra_loc += f;
+            if (cx(q)) m[0] += cx(q) * f;
+            if (cy(q)) m[1] += cy(q) * f;
+            if (cz(q)) m[2] += cz(q) * f;
         }
-        ra_loc[a] = r;
-        ma[a][0] = m0;
-        ma[a][1] = m1;
-        ma[a][2] = m2;
+        sh[RA + a][e] = ra_loc;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            sh[M + 3 * a + d][e] = m[d];
+            m[d] = ra_loc > 0.0 ? m[d] / ra_loc : 0.0;
+        }
+        sh[S + a][e] = m[0] * m[0] + m[1] * m[1] + m[2] * m[2];
     }
-    const GeqAxes<double> Gi = geq_axes<double>(th_in, vin);
+    double re_loc = 0;
+    if (on && energy) {
+        rho_t = R(TR_RHO);
+        th_t = R(TR_TH);
+        U_t = R(TR_U);
 #pragma unroll
-    for (int q = 0; q < Q; ++q)
-        re_loc += (unknown >> q & 1u) ? geq_dir<double>(Gi, q, rho_in, U_in - 1.5 * th_in) : ldg(v, v.g, q, c);
-    for (int a = 0; a < NS; ++a) {
-        rho_loc += ra_loc[a];
-        mloc[0] += ma[a][0];
-        mloc[1] += ma[a][1];
-        mloc[2] += ma[a][2];
+        for (int q = 0; q < Q; ++q) fin[q] = ldg(v, v.g, q, c);
+        const GeqAxes<double> Gt = geq_axes<double>(th_t, vt);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) ma[a][d] = ra_loc[a] > 0.0 ? ma[a][d] / ra_loc[a] : 0.0;
+        for (int q = 0; q < Q; ++q)
+            re_loc += (unknown >> q & 1u) ? geq_dir<double>(Gt, q, rho_t, U_t - 1.5 * th_t) : fin[q];
     }
-    double vloc[3];
+    __syncthreads();
+    // ---- mixture sums, calculate_temp (lbm-moment.cpp:540-553), local state
+    double rho_loc = 0, vloc[3], th_loc, U_loc, rho_g, th_g, U_g;
+    if (on && energy) {
+        double Yl[NS], mloc[3] = {0, 0, 0};
 #pragma unroll
-    for (int d = 0; d < 3; ++d) vloc[d] = rho_loc > 0 ? mloc[d] / rho_loc : 0.0;
-    double Uloc = re_loc / rho_loc;
-    for (int a = 0; a < NS; ++a)
-        Uloc = Uloc - 0.5 * ra_loc[a] / rho_loc * (ma[a][0] * ma[a][0] + ma[a][1] * ma[a][1] + ma[a][2] * ma[a][2]);
-    // calculate_temp (lbm-moment.cpp:540-553)
-    double Yl[NS];
+        for (int b = 0; b < NS; ++b) {
+            Yl[b] = sh[RA + b][e];
+            rho_loc += Yl[b];
 #pragma unroll
-    for (int a = 0; a < NS; ++a) Yl[a] = ra_loc[a] / rho_loc;
-    normalize(Yl);
-    const double T_loc = v.u.temp(T_from_UV(v.u.si_energy_mass(Uloc), Yl, v.u.si_temp(Fd[LBM_FIELD_T][c])));
-    const double Tsl = v.u.si_temp(T_loc);
-    const double U_loc = v.u.energy_mass(u_mass(Tsl, Yl));
-    const double th_loc = v.u.energy_mass(R_UNIV * Tsl / mean_W(Yl));
-    // target: local density and composition at the inflow velocity and temperature
-    const double U_tg = v.u.energy_mass(u_mass(Tsi, Yl));
-    const double th_tg = v.u.energy_mass(R_UNIV * Tsi / mean_W(Yl));
-    // ---- reconstruction
-    for (int a = 0; a < NS; ++a) {
-        const double thi = v.u.energy_mass(R_UNIV * Tsi / W[a]);
-        const double thl = v.u.energy_mass(R_UNIV * Tsl / W[a]);
-        Axis3<double> Fi[3], Fl[3];
-        feq_axes<double>(Fi, vin, thi, zero);
-        feq_axes<double>(Fl, ma[a], thl, zero);
+            for (int d = 0; d < 3; ++d) mloc[d] += sh[M + 3 * b + d][e];
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) vloc[d] = rho_loc > 0 ? mloc[d] / rho_loc : 0.0;
+        double Uloc = re_loc / rho_loc;
+#pragma unroll
+        for (int b = 0; b < NS; ++b) Uloc = Uloc - 0.5 * Yl[b] / rho_loc * sh[S + b][e];
+#pragma unroll
+        for (int b = 0; b < NS; ++b) Yl[b] = Yl[b] / rho_loc;
+        normalize(Yl);
+        const double T_loc =
+            v.u.temp(T_from_UV(v.u.si_energy_mass(Uloc), Yl, v.u.si_temp(v.fld[LBM_FIELD_T][c])));
+        const double Tsl = v.u.si_temp(T_loc);
+        sh[TSL][e] = Tsl;
+        U_loc = v.u.energy_mass(u_mass(Tsl, Yl));
+        th_loc = v.u.energy_mass(R_UNIV * Tsl / mean_W(Yl));
+        // the state a known direction is moved to: the target's, or at an inflow
+        // the local density and composition at the target velocity and temperature
+        rho_g = rho_t;
+        th_g = th_t;
+        U_g = U_t;
+        if (inflow) {
+            const double Ts = R(TR_TS);
+            rho_g = rho_loc;
+            U_g = v.u.energy_mass(u_mass(Ts, Yl));
+            th_g = v.u.energy_mass(R_UNIV * Ts / mean_W(Yl));
+        }
+    }
+    __syncthreads();
+    if (!on) return;
+    // ---- reconstruction: f_g + (unknown f_t, known f) - f_loc
+    if (!energy) {
+        const double thl = v.u.energy_mass(R_UNIV * sh[TSL][e] / W[a]);
+        Axis3<double> Ft[3], Fl[3];
+        feq_axes<double>(Ft, vt, th_t, zero);
+        feq_axes<double>(Fl, m, thl, zero);
+        const double ra_g = inflow ? ra_loc : rho_t;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const double fi = feq_dir<double>(Fi, q, ra_in[a]);
-            const double ft = feq_dir<double>(Fi, q, ra_loc[a]);
-            const double flc = feq_dir<double>(Fl, q, ra_loc[a]);
-            const double fin = ldf_in(v, a, q, c);
-            stf_in(v, a, q, c, (unknown >> q & 1u) ? ft + fi - flc : ft + fin - flc);
+            const double fg = feq_dir<double>(Ft, q, ra_g);
+            const double fl = feq_dir<double>(Fl, q, ra_loc);
+            const double f = (unknown >> q & 1u) ? feq_dir<double>(Ft, q, rho_t) : fin[q];
+            stf_in(v, a, q, c, fg + f - fl);
         }
+        return;
     }
+    const GeqAxes<double> Gt = geq_axes<double>(th_t, vt);
+    const GeqAxes<double> Gg = geq_axes<double>(th_g, vt);
     const GeqAxes<double> Gl = geq_axes<double>(th_loc, vloc);
-    const GeqAxes<double> Gt = geq_axes<double>(th_tg, vin);
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        const double gi = geq_dir<double>(Gi, q, rho_in, U_in - 1.5 * th_in);
-        const double gt = geq_dir<double>(Gt, q, rho_loc, U_tg - 1.5 * th_tg);
+        const double gg = geq_dir<double>(Gg, q, rho_g, U_g - 1.5 * th_g);
         const double gl = geq_dir<double>(Gl, q, rho_loc, U_loc - 1.5 * th_loc);
-        const double gin = ldg(v, v.g, q, c);
-        stg(v, v.g, q, c, (unknown >> q & 1u) ? gt + gi - gl : gt + gin - gl);
+        const double g = (unknown >> q & 1u) ? geq_dir<double>(Gt, q, rho_t, U_t - 1.5 * th_t) : fin[q];
+        stg(v, v.g, q, c, gg + g - gl);
     }
 }
 
@@ -2752,32 +2698,22 @@ void launch_mc(McKernel k, const MultiView<P>& v, hipStream_t s)
 }
 
 template <typename P>
-void launch_mc_tms(const MultiView<P>& v, const int* cells, const int* dirs, int count, double* rec, hipStream_t s)
+void launch_mc_tms(const MultiView<P>& v, const int* cells, const int* dirs, int n_out, int n_in, double* rec,
+                   hipStream_t s)
 {
     if constexpr (!kernels_built<P>()) {
         return;  // refused before launch (lbm_create, surrogate entry points)
     } else {
+        const int count = n_out + n_in;
         if (count <= 0) return;
-        const unsigned nb = (unsigned)((count + 63) / 64);
-        hipLaunchKernelGGL(k_mc_tms_target<P>, dim3(nb), dim3(64), 0, s, v, cells, dirs, count, rec);
-        hipLaunchKernelGGL(k_mc_tms_local<P>, dim3(nb, NS), dim3(64), 0, s, v, cells, count, rec);
-        hipLaunchKernelGGL(k_mc_tms_close<P>, dim3(nb), dim3(64), 0, s, v, cells, count, rec);
-        hipLaunchKernelGGL(k_mc_tms_rebuild<P>, dim3(nb, NS + 1), dim3(64), 0, s, v, cells, count,
-                           static_cast<const double*>(rec));
+        hipLaunchKernelGGL(k_mc_tms_target<P>, dim3((n_out + 63) / 64 + (n_in + 63) / 64), dim3(64), 0, s, v, cells, dirs,
+                           n_out, n_in, rec);
+        hipLaunchKernelGGL(k_mc_tms_sweep<P>, dim3((count + TMS_E - 1) / TMS_E), dim3(TMS_ROW + 64), 0, s, v, cells,
+                           n_out, count, static_cast<const double*>(rec));
     }
 }
 
 int mc_tms_record_fields() { return TR_COUNT; }
-
-template <typename P>
-void launch_mc_tms_in(const MultiView<P>& v, const int* cells, const int* dirs, int count, hipStream_t s)
-{
-    if constexpr (!kernels_built<P>()) {
-        return;  // refused before launch (lbm_create, surrogate entry points)
-    } else {
-        if (count > 0) hipLaunchKernelGGL(k_mc_tms_in<P>, dim3((count + 63) / 64), dim3(64), 0, s, v, cells, dirs, count);
-    }
-}
 
 template <typename P>
 void launch_mc_tms_wall(const MultiView<P>& v, const int* cells, int count, hipStream_t s)
@@ -2894,17 +2830,15 @@ template void launch_mc_aa_save<double>(const MultiView<double>&, bool, int, int
 template void launch_mc_aa_save<float>(const MultiView<float>&, bool, int, int, hipStream_t);
 template void launch_mc_aa_collide<double>(const MultiView<double>&, int, int, bool, hipStream_t);
 template void launch_mc_aa_collide<float>(const MultiView<float>&, int, int, bool, hipStream_t);
-template void launch_mc_tms<float>(const MultiView<float>&, const int*, const int*, int, double*, hipStream_t);
+template void launch_mc_tms<float>(const MultiView<float>&, const int*, const int*, int, int, double*, hipStream_t);
 template void launch_mc_sur_chemistry<float>(const MultiView<float>&, const sur::Mlp&, unsigned*, unsigned*,
                                              hipStream_t);
 template void launch_mc_chem_list<float>(const MultiView<float>&, const unsigned*, const unsigned*, hipStream_t);
 template void launch_mc_sur_chemistry<double>(const MultiView<double>&, const sur::Mlp&, unsigned*, unsigned*,
                                               hipStream_t);
 template void launch_mc_chem_list<double>(const MultiView<double>&, const unsigned*, const unsigned*, hipStream_t);
-template void launch_mc_tms<double>(const MultiView<double>&, const int*, const int*, int, double*, hipStream_t);
-template void launch_mc_tms_in<double>(const MultiView<double>&, const int*, const int*, int, hipStream_t);
+template void launch_mc_tms<double>(const MultiView<double>&, const int*, const int*, int, int, double*, hipStream_t);
 template void launch_mc_tms_wall<double>(const MultiView<double>&, const int*, int, hipStream_t);
 template void launch_mc_tms_wall<float>(const MultiView<float>&, const int*, int, hipStream_t);
-template void launch_mc_tms_in<float>(const MultiView<float>&, const int*, const int*, int, hipStream_t);
 
 }  // namespace lbm
