@@ -2232,7 +2232,7 @@ void train_release(lbm_ctx* c)
 
 // Enqueues `iters` training iterations of `net` on stream st, from the first
 // `rows` capture rows normalised by `stats`, with Adam steps adam_step + 1 ...
-// One iteration (batch draw, forward and backward passes, loss, Adam: 45
+// One iteration (batch draw, gradient, loss, Adam: 17
 // kernels) is captured once as a HIP graph and replayed `iters` times; the
 // iteration index and the step's Adam corrections are read on the device.
 // The graph is kept in c->tgraph / c->texec until train_release, after st
@@ -2581,9 +2581,8 @@ int lbm_surrogate_gradient(lbm_ctx* c, const float* X, const float* T, int64_t m
         HIP_TRY(c, hipMalloc((void**)&c->bloss, sizeof(float)));
         c->lcap = 1;
     }
-    float* xf = nullptr;
+    float* const xf = c->work.xf;
     const size_t bytes = sizeof(float) * 16 * (size_t)m;
-    HIP_TRY(c, hipMalloc((void**)&xf, bytes));
     hipError_t e = hipMemcpyAsync(xf, X, bytes, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(c->bt, T, bytes, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) {
@@ -2592,16 +2591,10 @@ int lbm_surrogate_gradient(lbm_ctx* c, const float* X, const float* T, int64_t m
         sur::loss_sum(c->work.loss_rows, (int)m, 1.f / ((float)m * sur::NOUT), c->bloss, c->stream);
         e = hipGetLastError();
     }
-    size_t off = 0;
-    for (int L = 0; L < sur::NL && e == hipSuccess; ++L) {
-        const size_t nw = (size_t)sur::DIMS[L] * sur::DIMS[L + 1], nb = sur::DIMS[L + 1];
-        e = hipMemcpyAsync(grad + off, c->work.gW[L], 4 * nw, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(grad + off + nw, c->work.gb[L], 4 * nb, hipMemcpyDeviceToHost, c->stream);
-        off += nw + nb;
-    }
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(grad, c->work.grad, sizeof(float) * sur::NPARAM, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(loss, c->bloss, sizeof(float), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(xf);
     if (e != hipSuccess) return fail(c, LBM_E_HIP, std::string("surrogate gradient: ") + hipGetErrorString(e));
     return LBM_OK;
 }

@@ -25,16 +25,14 @@ struct Mlp {
     uint16_t* Wf = nullptr;  // all layers in MFMA fragment order (in-step inference)
 };
 
-// Activations and gradient scratch for batches of up to `cap` rows.
+// Gradient scratch for batches of up to `cap` rows.
 struct Work {
-    int cap = 0, chunk = 256;
-    float* Z[NL] = {};
-    uint16_t* H[NL] = {};
-    uint16_t* dZ[NL] = {};
-    uint16_t *dZT = nullptr, *XT = nullptr;
-    float* part = nullptr;
-    float *gW[NL] = {}, *gb[NL] = {};
+    int cap = 0;
+    float* part = nullptr;  // the blocks' shares of the flat gradient
+    float* grad = nullptr;  // flat gradient [NPARAM]: W[0], b[0], W[1], ...
+    float *gW[NL] = {}, *gb[NL] = {};  // its parts
     float* loss_rows = nullptr;
+    float* xf = nullptr;  // [cap][16] FP32 features of a caller's batch
 };
 
 // Capture rows [rows][32]: raw features T [K], p [Pa], Y_k (NS), dt [s], zero
@@ -54,10 +52,8 @@ hipError_t work_alloc(Work& w, int cap);
 void work_free(Work& w);
 void refresh_bf16(Mlp& net, hipStream_t s);
 void to_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t s);
-// Forward pass of M rows (M multiple of 16); the outputs are w.Z[NL-1] [M][16].
-void mlp_forward(const Mlp& net, const uint16_t* X, int M, Work& w, hipStream_t s);
 // Gradients of the mean-squared loss over the NOUT outputs for one batch (M
-// multiple of 16) into w.gW / w.gb; per-row losses land in w.loss_rows.
+// multiple of 16, at most w.cap) into w.grad; per-row losses land in w.loss_rows.
 void mlp_grad(const Mlp& net, const uint16_t* X, const float* T, int M, Work& w, hipStream_t s);
 // One Adam step with the gradients in w; the bias corrections of the step are
 // c12[2 *it], c12[2 *it + 1] (device), filled by adam_corrections (host) for

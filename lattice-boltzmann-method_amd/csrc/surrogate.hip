@@ -3,10 +3,7 @@
 // FP32 accumulation, Adam on FP32 master weights.
 //
 // Layers: 16 (NIN = NS + 3 features, zero-padded) -> 128 -> 128 -> 128 -> 16
-// (NOUT = NS + 1 outputs, zero-padded), GELU (tanh form) on the hidden layers.  Every training GEMM is
-// C[m][n] = sum_k A[m][k] B[n][k] (+ bias) on 16x16 output tiles, one
-// wavefront per tile, v_mfma_f32_16x16x16_bf16 with 4 BF16 of A and of B per
-// lane per K-step of 16 (operand layout in surrogate_device.h).
+// (NOUT = NS + 1 outputs, zero-padded), GELU (tanh form) on the hidden layers.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -19,144 +16,265 @@
 namespace lbm {
 namespace sur {
 
-// One 16x16 tile of C = A B^T with A [M][lda] and B [N][ldb] in BF16 (K
-// multiple of 16, M and N multiples of 16).
-__device__ inline v4f tile_mma(const uint16_t* A, int lda, const uint16_t* B, int ldb, int m0, int n0, int K)
+// ------------------------------------------------------- gradient kernel
+// Forward pass, loss and all gradients of the batch in one pass over its rows:
+// a block takes GROWS rows at a time through the four layers and back and keeps
+// its weight gradients in registers.  One wavefront per 16 neurons of the
+// 128-wide layers: with Z^T = W H^T (A operand the weights, i = neuron; B
+// operand the batch rows) the pre-activations a wavefront makes going forward
+// are in its own registers, in place, when the backward pass wants gelu' of
+// them.  Activations and dZ pass between wavefronts as BF16 in LDS, by row for
+// the next layer's product and transposed for the weight gradients, whose
+// reduction index is the row; both strides spread 16 rows of 16 bytes over all
+// banks.  Weights are read where they are used (72 KiB from L2).
+// Bound by the chain of eight phases between barriers.  With a pass per layer
+// and operand (forward, transposes, partial products, their sums, bias sums:
+// 33 launches) a caller's gradient of 4096 rows took 395 us, host copies
+// included, and takes 127.
+constexpr int GWAVES = 8, GROWS = 64, GTILES = GROWS / 16, GSTEPS = GROWS / 32;
+constexpr int GRAD_BLOCKS = 256;       // one per CU: more rows go round
+constexpr int HSTRIDE = 128 + 8, TSTRIDE = GROWS + 8, DSTRIDE = 16 + 8;
+static_assert(GWAVES * 16 == 128, "one wavefront per 16 neurons");
+
+// Offsets of W[L] and b[L] in the flat gradient.
+constexpr int grad_w(int L) { return frag_offset(L) + bias_offset(L); }
+constexpr int grad_b(int L) { return grad_w(L) + DIMS[L] * DIMS[L + 1]; }
+static_assert(grad_b(NL - 1) + DIMS[NL] == NPARAM, "flat gradient");
+
+// Four neurons n0 + 0..3 of row r, by row and transposed.
+__device__ __forceinline__ void put_rows(uint16_t* h, int r, int n0, const v4s x)
+{
+    uint2 u;
+    __builtin_memcpy(&u, &x, 8);
+    *reinterpret_cast<uint2*>(h + r * HSTRIDE + n0) = u;
+}
+__device__ __forceinline__ void put_cols(uint16_t* hT, int r, int n0, const v4s x)
+{
+#pragma unroll
+    for (int q = 0; q < 4; ++q) hT[(n0 + q) * TSTRIDE + r] = (uint16_t)x[q];
+}
+// acc += A[16 a0 + ..][rows] B[16 b0 + ..][rows]^T over the block's rows
+__device__ __forceinline__ v4f row_products(const v8bf a[GSTEPS], const uint16_t* bT, int b0, v4f acc)
 {
     const int lane = threadIdx.x & 63;
-    const int r = lane & 15, kq = (lane >> 4) * 4;
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        const uint16_t* pa = A + (size_t)(m0 + r) * lda + k0 + kq;
-        const uint16_t* pb = B + (size_t)(n0 + r) * ldb + k0 + kq;
-        v4s a, b;
-        a[0] = (short)pa[0]; a[1] = (short)pa[1]; a[2] = (short)pa[2]; a[3] = (short)pa[3];
-        b[0] = (short)pb[0]; b[1] = (short)pb[1]; b[2] = (short)pb[2]; b[3] = (short)pb[3];
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-    }
+#pragma unroll
+    for (int s = 0; s < GSTEPS; ++s)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            a[s], load_frag8(bT + (16 * b0 + (lane & 15)) * TSTRIDE + 32 * s + 8 * (lane >> 4)), acc, 0, 0, 0);
     return acc;
 }
-
-// Layer forward: Z = X W^T + b (FP32, kept for the backward), H = act(Z) in
-// BF16 for the next layer.  Grid: x = M/16 row tiles, y = N/16 column tiles
-// (one wavefront per tile, 64 threads per block).
-__global__ __launch_bounds__(64) void k_layer_fwd(const uint16_t* X, int K, const uint16_t* W, const float* b, int N,
-                                                  float* Z, uint16_t* H, int act, int M)
+__device__ __forceinline__ void row_operand(const uint16_t* aT, int a0, v8bf a[GSTEPS])
 {
-    const int m0 = blockIdx.x * 16, n0 = blockIdx.y * 16;
-    if (m0 >= M) return;
-    const v4f acc = tile_mma(X, K, W, K, m0, n0, K);
     const int lane = threadIdx.x & 63;
-    const int col = n0 + (lane & 15);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int row = m0 + (lane >> 4) * 4 + v;
-        const float z = acc[v] + b[col];
-        if (Z) Z[(size_t)row * N + col] = z;
-        if (H) H[(size_t)row * N + col] = f2bf(act ? gelu(z) : z);
+    for (int s = 0; s < GSTEPS; ++s)
+        a[s] = load_frag8(aT + (16 * a0 + (lane & 15)) * TSTRIDE + 32 * s + 8 * (lane >> 4));
+}
+// sum over the block's rows of A: the product with ones
+__device__ __forceinline__ v4f row_sums(const v8bf a[GSTEPS], v4f acc)
+{
+    v8bf one;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) one[e] = (__bf16)1.0f;
+#pragma unroll
+    for (int s = 0; s < GSTEPS; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], one, acc, 0, 0, 0);
+    return acc;
+}
+// out[bt] = W[16 w0 + ..][0..128) h[row][0..128)^T for the block's row tiles
+__device__ __forceinline__ void product128(const uint16_t* W, int w0, const uint16_t* h, v4f out[GTILES])
+{
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    v8bf a[KSTEPS];
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) a[s] = load_frag8(W + (16 * w0 + j) * 128 + 32 * s + 8 * g);
+#pragma unroll
+    for (int bt = 0; bt < GTILES; ++bt) {
+        out[bt] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+            out[bt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                a[s], load_frag8(h + (16 * bt + j) * HSTRIDE + 32 * s + 8 * g), out[bt], 0, 0, 0);
     }
 }
-
-// dZ of the output layer for the mean-squared loss over `nout` outputs:
-// dZ = 2 (z - t) / (M nout); padded outputs get 0.  Also the per-row loss.
-__global__ void k_loss_grad(const float* Z, const float* T, int M, int N, int nout, uint16_t* dZb, float* loss_rows)
+__device__ __forceinline__ v4s bf_frag(const v4f z)
 {
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= M) return;
-    float s = 0.f;
-    for (int c = 0; c < N; ++c) {
-        float g = 0.f;
-        if (c < nout) {
-            const float d = Z[(size_t)row * N + c] - T[(size_t)row * N + c];
-            s += d * d;
-            g = 2.f * d / (float)(M * nout);
+    v4s r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = (short)f2bf(z[q]);
+    return r;
+}
+
+// grid: at most GRAD_BLOCKS blocks of 64 GWAVES threads, M a multiple of 16;
+// part [gridDim.x][NPARAM] receives each block's share of the flat gradient,
+// loss_rows [M] the rows' squared errors.  dZ of the output layer is that of
+// the mean-squared loss over NOUT outputs, 2 (z - t) / (M NOUT), and 0 for
+// padded outputs and for rows past M.
+__global__ __launch_bounds__(64 * GWAVES) void k_grad(Mlp net, const uint16_t* X, const float* T, int M, float* part,
+                                                      float* loss_rows)
+{
+    __shared__ __align__(16) uint16_t h[2][GROWS * HSTRIDE];   // by row: activations, then dZ
+    __shared__ __align__(16) uint16_t hT[3][128 * TSTRIDE];    // transposed activations
+    __shared__ __align__(16) uint16_t dT[2][128 * TSTRIDE];    // transposed dZ
+    __shared__ __align__(16) uint16_t xT[16 * TSTRIDE], d3T[16 * TSTRIDE], d3[GROWS * DSTRIDE];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
+    const int n0 = 16 * w + 4 * g;  // the neurons of this lane's D fragments
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    v4f g0 = zero, g1[8], g2[8], g3 = zero, s0 = zero, s1 = zero, s2 = zero, s3 = zero;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) g1[t] = g2[t] = zero;
+    for (int r0 = blockIdx.x * GROWS; r0 < M; r0 += gridDim.x * GROWS) {
+        v4f z0[GTILES], z1[GTILES], z2[GTILES], acc[GTILES];
+        v8bf a[GSTEPS];
+        {  // ---- layer 0, K = 16
+            const v4s wf = load_frag(net.Wb[0] + (16 * w + j) * 16 + 4 * g);
+            const v4f b = bias_frag(net.b[0], 16 * w, lane);
+#pragma unroll
+            for (int bt = 0; bt < GTILES; ++bt) {
+                const int r = 16 * bt + j;
+                v4s x = {0, 0, 0, 0};
+                if (r0 + r < M) x = load_frag(X + (size_t)(r0 + r) * 16 + 4 * g);
+                if (w == bt) put_cols(xT, r, 4 * g, x);
+                z0[bt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wf, x, zero, 0, 0, 0) + b;
+                const v4s hf = act_frag(z0[bt]);
+                put_rows(h[0], r, n0, hf);
+                put_cols(hT[0], r, n0, hf);
+            }
         }
-        dZb[(size_t)row * N + c] = f2bf(g);
-    }
-    loss_rows[row] = s;
-}
-
-// dX = dZ W (rows of W^T given as WT [K][N]); then for a hidden layer below,
-// dZ_below = dX * gelu'(Z_below).
-__global__ __launch_bounds__(64) void k_layer_bwd_x(const uint16_t* dZ, int N, const uint16_t* WT, int K,
-                                                    const float* Zbelow, uint16_t* dZbelow, int M)
-{
-    const int m0 = blockIdx.x * 16, k0 = blockIdx.y * 16;
-    if (m0 >= M) return;
-    const v4f acc = tile_mma(dZ, N, WT, N, m0, k0, N);
-    const int lane = threadIdx.x & 63;
-    const int col = k0 + (lane & 15);
+        __syncthreads();
+        // ---- layers 1 and 2
+        auto hidden = [&](int L, const uint16_t* from, uint16_t* to, uint16_t* toT, v4f z[GTILES]) {
+            product128(net.Wb[L], w, from, z);
+            const v4f b = bias_frag(net.b[L], 16 * w, lane);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int row = m0 + (lane >> 4) * 4 + v;
-        const float g = acc[v] * gelu_grad(Zbelow[(size_t)row * K + col]);
-        dZbelow[(size_t)row * K + col] = f2bf(g);
-    }
-}
-
-// Transposes a BF16 [M][N] matrix into [N][M] (for the weight gradient the
-// batch is the reduction index): 64 x 64 tiles through LDS, so that the
-// reads run along rows of `in` and the writes along rows of `out`.
-// grid (ceil(M / 64), ceil(N / 64)), 256 threads.
-__global__ __launch_bounds__(256) void k_transpose_bf(const uint16_t* in, int M, int N, uint16_t* out)
-{
-    __shared__ uint16_t tile[64][65];
-    const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int r = ty; r < 64; r += 4) {
-        const int m = m0 + r, n = n0 + tx;
-        tile[r][tx] = (m < M && n < N) ? in[(size_t)m * N + n] : (uint16_t)0;
-    }
-    __syncthreads();
-    for (int r = ty; r < 64; r += 4) {
-        const int n = n0 + r, m = m0 + tx;
-        if (n < N && m < M) out[(size_t)n * M + m] = tile[tx][r];
-    }
-}
-
-// Partial weight gradient over one chunk of rows: dW[n][k] = sum_m dZ[m][n] X[m][k]
-// with dZT [N][M] and XT [K][M]; chunk c covers rows [c*chunk, (c+1)*chunk).
-__global__ __launch_bounds__(64) void k_wgrad(const uint16_t* dZT, const uint16_t* XT, int M, int N, int K, int chunk,
-                                              float* part)
-{
-    const int n0 = blockIdx.x * 16, k0 = blockIdx.y * 16, c = blockIdx.z;
-    const int mbeg = c * chunk;
-    const int len = min(chunk, M - mbeg);
-    const v4f acc = tile_mma(dZT + mbeg, M, XT + mbeg, M, n0, k0, len);
-    const int lane = threadIdx.x & 63;
-    const int col = k0 + (lane & 15);
+            for (int bt = 0; bt < GTILES; ++bt) {
+                z[bt] += b;
+                const v4s hf = act_frag(z[bt]);
+                put_rows(to, 16 * bt + j, n0, hf);
+                put_cols(toT, 16 * bt + j, n0, hf);
+            }
+        };
+        hidden(1, h[0], h[1], hT[1], z1);
+        __syncthreads();
+        hidden(2, h[1], h[0], hT[2], z2);
+        __syncthreads();
+        // ---- output layer and loss: row tile w
+        if (w < GTILES) {
+            const int r = 16 * w + j, row = r0 + r;
+            v4f z = zero;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int row = n0 + (lane >> 4) * 4 + v;
-        part[((size_t)c * N + row) * K + col] = acc[v];
-    }
-}
-
-// Sums the chunk partials in a fixed order (deterministic).
-__global__ void k_reduce_grad(const float* part, int nchunk, int N, int K, float* dW)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N * K) return;
-    float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += part[(size_t)c * N * K + i];
-    dW[i] = s;
-}
-
-// Bias gradient db[n] = sum_m dZ[m][n]: one block per n, strided partial
-// sums reduced in LDS in a fixed order.
-__global__ __launch_bounds__(256) void k_bias_grad(const uint16_t* dZT, int M, float* db)
-{
-    __shared__ float red[256];
-    const int nrow = blockIdx.x;
-    float s = 0.f;
-    for (int m = threadIdx.x; m < M; m += 256) s += bf2f(dZT[(size_t)nrow * M + m]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+            for (int s = 0; s < KSTEPS; ++s)
+                z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_frag8(net.Wb[3] + j * 128 + 32 * s + 8 * g),
+                                                           load_frag8(h[0] + r * HSTRIDE + 32 * s + 8 * g), z, 0, 0, 0);
+            z += bias_frag(net.b[3], 0, lane);
+            v4f dz = zero;
+            float sum = 0.f;
+            if (row < M) {
+                const v4f t = *reinterpret_cast<const v4f*>(T + (size_t)row * 16 + 4 * g);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (4 * g + q < NOUT) {
+                        const float d = z[q] - t[q];
+                        sum += d * d;
+                        dz[q] = 2.f * d / (float)(M * NOUT);
+                    }
+            }
+            sum += __shfl_xor(sum, 16);
+            sum += __shfl_xor(sum, 32);
+            if (g == 0 && row < M) loss_rows[row] = sum;
+            const v4s df = bf_frag(dz);
+            uint2 u;
+            __builtin_memcpy(&u, &df, 8);
+            *reinterpret_cast<uint2*>(d3 + r * DSTRIDE + 4 * g) = u;
+            put_cols(d3T, r, 4 * g, df);
+        }
+        __syncthreads();
+        // ---- back through the output layer; its weight gradient
+        {
+            const v4s wf = load_frag(net.WbT[3] + (16 * w + j) * 16 + 4 * g);
+#pragma unroll
+            for (int bt = 0; bt < GTILES; ++bt) {
+                const int r = 16 * bt + j;
+                v4f d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wf, load_frag(d3 + r * DSTRIDE + 4 * g), zero, 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) d[q] *= gelu_grad(z2[bt][q]);
+                const v4s df = bf_frag(d);
+                put_rows(h[1], r, n0, df);
+                put_cols(dT[0], r, n0, df);
+            }
+            row_operand(d3T, 0, a);
+            g3 = row_products(a, hT[2], w, g3);
+            s3 = row_sums(a, s3);
+        }
+        __syncthreads();
+        // ---- layer 2
+        product128(net.WbT[2], w, h[1], acc);
+#pragma unroll
+        for (int bt = 0; bt < GTILES; ++bt) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[bt][q] *= gelu_grad(z1[bt][q]);
+            const v4s df = bf_frag(acc[bt]);
+            put_rows(h[0], 16 * bt + j, n0, df);
+            put_cols(dT[1], 16 * bt + j, n0, df);
+        }
+        row_operand(dT[0], w, a);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) g2[t] = row_products(a, hT[1], t, g2[t]);
+        s2 = row_sums(a, s2);
+        __syncthreads();
+        // ---- layer 1
+        product128(net.WbT[1], w, h[0], acc);
+#pragma unroll
+        for (int bt = 0; bt < GTILES; ++bt) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[bt][q] *= gelu_grad(z0[bt][q]);
+            put_cols(dT[0], 16 * bt + j, n0, bf_frag(acc[bt]));
+        }
+        row_operand(dT[1], w, a);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) g1[t] = row_products(a, hT[0], t, g1[t]);
+        s1 = row_sums(a, s1);
+        __syncthreads();
+        // ---- layer 0
+        row_operand(dT[0], w, a);
+        g0 = row_products(a, xT, 0, g0);
+        s0 = row_sums(a, s0);
         __syncthreads();
     }
-    if (threadIdx.x == 0) db[nrow] = red[0];
+    // ---- the block's share, in the flat order
+    float* out = part + (size_t)blockIdx.x * NPARAM;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        out[grad_w(0) + (n0 + q) * 16 + j] = g0[q];
+        out[grad_w(3) + (4 * g + q) * 128 + 16 * w + j] = g3[q];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            out[grad_w(1) + (n0 + q) * 128 + 16 * t + j] = g1[t][q];
+            out[grad_w(2) + (n0 + q) * 128 + 16 * t + j] = g2[t][q];
+        }
+        if (j == 0) {
+            out[grad_b(0) + n0 + q] = s0[q];
+            out[grad_b(1) + n0 + q] = s1[q];
+            out[grad_b(2) + n0 + q] = s2[q];
+            if (w == 0) out[grad_b(3) + 4 * g + q] = s3[q];
+        }
+    }
+}
+
+// Sums the blocks' shares in a fixed order: 64 parameters per block of 256, a
+// quarter of the shares per wavefront.
+__global__ __launch_bounds__(256) void k_grad_sum(const float* part, int nblk, float* grad)
+{
+    __shared__ float red[4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
+    float s = 0.f;
+    if (i < NPARAM) {
+#pragma unroll 8
+        for (int b = w; b < nblk; b += 4) s += part[(size_t)b * NPARAM + i];
+    }
+    red[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && i < NPARAM) grad[i] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
 // Adam on FP32 master weights; refreshes the BF16 copies W and W^T.  The
@@ -405,38 +523,13 @@ void loss_sum(const float* loss_rows, int B, float scale, float* out, hipStream_
     hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(256), 0, s, loss_rows, B, scale, out, idx);
 }
 
-void mlp_forward(const Mlp& net, const uint16_t* X, int M, Work& w, hipStream_t s)
-{
-    const uint16_t* in = X;
-    for (int L = 0; L < NL; ++L) {
-        const int K = DIMS[L], N = DIMS[L + 1];
-        const bool last = (L == NL - 1);
-        hipLaunchKernelGGL(k_layer_fwd, dim3(M / 16, N / 16), dim3(64), 0, s, in, K, net.Wb[L], net.b[L], N, w.Z[L],
-                           last ? (uint16_t*)nullptr : w.H[L], last ? 0 : 1, M);
-        in = w.H[L];
-    }
-}
+static int grad_blocks(int M) { return cdiv(M, GROWS) < GRAD_BLOCKS ? cdiv(M, GROWS) : GRAD_BLOCKS; }
 
 void mlp_grad(const Mlp& net, const uint16_t* X, const float* T, int M, Work& w, hipStream_t s)
 {
-    mlp_forward(net, X, M, w, s);
-    const int L3 = NL - 1;
-    hipLaunchKernelGGL(k_loss_grad, dim3(cdiv(M, 256)), dim3(256), 0, s, w.Z[L3], T, M, DIMS[NL], NOUT, w.dZ[L3],
-                       w.loss_rows);
-    for (int L = NL - 1; L >= 0; --L) {
-        const int K = DIMS[L], N = DIMS[L + 1];
-        const uint16_t* Xin = L == 0 ? X : w.H[L - 1];
-        hipLaunchKernelGGL(k_transpose_bf, dim3(cdiv(M, 64), cdiv(N, 64)), dim3(256), 0, s, w.dZ[L], M, N, w.dZT);
-        hipLaunchKernelGGL(k_transpose_bf, dim3(cdiv(M, 64), cdiv(K, 64)), dim3(256), 0, s, Xin, M, K, w.XT);
-        const int nchunk = cdiv(M, w.chunk);
-        hipLaunchKernelGGL(k_wgrad, dim3(N / 16, K / 16, nchunk), dim3(64), 0, s, w.dZT, w.XT, M, N, K, w.chunk,
-                           w.part);
-        hipLaunchKernelGGL(k_reduce_grad, dim3(cdiv(N * K, 256)), dim3(256), 0, s, w.part, nchunk, N, K, w.gW[L]);
-        hipLaunchKernelGGL(k_bias_grad, dim3(N), dim3(256), 0, s, w.dZT, M, w.gb[L]);
-        if (L > 0)
-            hipLaunchKernelGGL(k_layer_bwd_x, dim3(M / 16, K / 16), dim3(64), 0, s, w.dZ[L], N, net.WbT[L], K,
-                               w.Z[L - 1], w.dZ[L - 1], M);
-    }
+    const int nblk = grad_blocks(M);
+    hipLaunchKernelGGL(k_grad, dim3(nblk), dim3(64 * GWAVES), 0, s, net, X, T, M, w.part, w.loss_rows);
+    hipLaunchKernelGGL(k_grad_sum, dim3(cdiv(NPARAM, 64)), dim3(256), 0, s, w.part, nblk, w.grad);
 }
 
 void adam_corrections(int first_step, int iters, float* c12)
@@ -581,32 +674,20 @@ hipError_t work_alloc(Work& w, int cap)
 {
     hipError_t e;
     w.cap = cap;
-    int maxd = 0;
-    for (int L = 0; L <= NL; ++L) maxd = DIMS[L] > maxd ? DIMS[L] : maxd;
-    for (int L = 0; L < NL; ++L) {
-        const int N = DIMS[L + 1];
-        if ((e = hipMalloc((void**)&w.Z[L], sizeof(float) * (size_t)cap * N)) != hipSuccess) return e;
-        if ((e = hipMalloc((void**)&w.H[L], 2 * (size_t)cap * N)) != hipSuccess) return e;
-        if ((e = hipMalloc((void**)&w.dZ[L], 2 * (size_t)cap * N)) != hipSuccess) return e;
-        if ((e = hipMalloc((void**)&w.gW[L], sizeof(float) * DIMS[L] * N)) != hipSuccess) return e;
-        if ((e = hipMalloc((void**)&w.gb[L], sizeof(float) * N)) != hipSuccess) return e;
-    }
-    if ((e = hipMalloc((void**)&w.dZT, 2 * (size_t)cap * maxd)) != hipSuccess) return e;
-    if ((e = hipMalloc((void**)&w.XT, 2 * (size_t)cap * maxd)) != hipSuccess) return e;
-    const int nchunk = (cap + w.chunk - 1) / w.chunk;
-    if ((e = hipMalloc((void**)&w.part, sizeof(float) * (size_t)nchunk * maxd * maxd)) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&w.part, sizeof(float) * NPARAM * (size_t)grad_blocks(cap))) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&w.grad, sizeof(float) * NPARAM)) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&w.loss_rows, sizeof(float) * (size_t)cap)) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&w.xf, sizeof(float) * 16 * (size_t)cap)) != hipSuccess) return e;
+    for (int L = 0; L < NL; ++L) {
+        w.gW[L] = w.grad + grad_w(L);
+        w.gb[L] = w.grad + grad_b(L);
+    }
     return hipSuccess;
 }
 
 void work_free(Work& w)
 {
-    for (int L = 0; L < NL; ++L) {
-        void* ps[] = {w.Z[L], w.H[L], w.dZ[L], w.gW[L], w.gb[L]};
-        for (void* p : ps)
-            if (p) (void)hipFree(p);
-    }
-    void* ps[] = {w.dZT, w.XT, w.part, w.loss_rows};
+    void* ps[] = {w.part, w.grad, w.loss_rows, w.xf};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     w = Work{};
