@@ -2089,6 +2089,7 @@ int sur_batch(lbm_ctx* c, int rows)
     if (c->bt) (void)hipFree(c->bt);
     c->bx = nullptr;
     c->bt = nullptr;
+    c->bcap = 0;
     HIP_TRY(c, hipMalloc((void**)&c->bx, sizeof(uint16_t) * 16 * (size_t)rows));
     HIP_TRY(c, hipMalloc((void**)&c->bt, sizeof(float) * 16 * (size_t)rows));
     c->bcap = rows;
@@ -2214,6 +2215,7 @@ int train_buffers(lbm_ctx* c, int iters, int batch)
         if (c->adam_c12) (void)hipFree(c->adam_c12);
         c->bloss = nullptr;
         c->adam_c12 = nullptr;
+        c->lcap = 0;
         HIP_TRY(c, hipMalloc((void**)&c->bloss, sizeof(float) * std::max(iters, 1)));
         HIP_TRY(c, hipMalloc((void**)&c->adam_c12, sizeof(float) * 2 * std::max(iters, 1)));
         c->lcap = std::max(iters, 1);

@@ -48,6 +48,7 @@ hipError_t mlp_alloc(Mlp& net, uint64_t seed, hipStream_t s);
 hipError_t mlp_alloc_empty(Mlp& net);
 hipError_t mlp_copy(Mlp& dst, const Mlp& src, hipStream_t s);
 void mlp_free(Mlp& net);
+// (a failure leaves w empty, cap 0)
 hipError_t work_alloc(Work& w, int cap);
 void work_free(Work& w);
 void refresh_bf16(Mlp& net, hipStream_t s);

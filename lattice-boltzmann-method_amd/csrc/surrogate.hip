@@ -670,18 +670,22 @@ void mlp_free(Mlp& net)
     net = Mlp{};
 }
 
+// (cap is set once everything is there: a caller asks it whether to allocate)
 hipError_t work_alloc(Work& w, int cap)
 {
-    hipError_t e;
-    w.cap = cap;
-    if ((e = hipMalloc((void**)&w.part, sizeof(float) * NPARAM * (size_t)grad_blocks(cap))) != hipSuccess) return e;
-    if ((e = hipMalloc((void**)&w.grad, sizeof(float) * NPARAM)) != hipSuccess) return e;
-    if ((e = hipMalloc((void**)&w.loss_rows, sizeof(float) * (size_t)cap)) != hipSuccess) return e;
-    if ((e = hipMalloc((void**)&w.xf, sizeof(float) * 16 * (size_t)cap)) != hipSuccess) return e;
+    hipError_t e = hipMalloc((void**)&w.part, sizeof(float) * NPARAM * (size_t)grad_blocks(cap));
+    if (e == hipSuccess) e = hipMalloc((void**)&w.grad, sizeof(float) * NPARAM);
+    if (e == hipSuccess) e = hipMalloc((void**)&w.loss_rows, sizeof(float) * (size_t)cap);
+    if (e == hipSuccess) e = hipMalloc((void**)&w.xf, sizeof(float) * 16 * (size_t)cap);
+    if (e != hipSuccess) {
+        work_free(w);
+        return e;
+    }
     for (int L = 0; L < NL; ++L) {
         w.gW[L] = w.grad + grad_w(L);
         w.gb[L] = w.grad + grad_b(L);
     }
+    w.cap = cap;
     return hipSuccess;
 }
 
