@@ -2234,7 +2234,7 @@ void train_release(lbm_ctx* c)
 
 // Enqueues `iters` training iterations of `net` on stream st, from the first
 // `rows` capture rows normalised by `stats`, with Adam steps adam_step + 1 ...
-// One iteration (batch draw, gradient, loss, Adam: 17
+// One iteration (batch draw, gradient, loss, Adam: 18
 // kernels) is captured once as a HIP graph and replayed `iters` times; the
 // iteration index and the step's Adam corrections are read on the device.
 // The graph is kept in c->tgraph / c->texec until train_release, after st
@@ -2588,8 +2588,7 @@ int lbm_surrogate_gradient(lbm_ctx* c, const float* X, const float* T, int64_t m
     hipError_t e = hipMemcpyAsync(xf, X, bytes, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(c->bt, T, bytes, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) {
-        sur::to_bf16(xf, c->bx, 16 * m, c->stream);
-        sur::mlp_grad(c->net, c->bx, c->bt, (int)m, c->work, c->stream);
+        sur::mlp_grad(c->net, xf, c->bt, (int)m, c->work, c->stream);
         sur::loss_sum(c->work.loss_rows, (int)m, 1.f / ((float)m * sur::NOUT), c->bloss, c->stream);
         e = hipGetLastError();
     }

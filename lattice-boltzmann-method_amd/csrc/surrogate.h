@@ -28,7 +28,8 @@ struct Mlp {
 // Gradient scratch for batches of up to `cap` rows.
 struct Work {
     int cap = 0;
-    float* part = nullptr;  // the blocks' shares of the flat gradient
+    uint16_t* tiles = nullptr;  // transposed activations and dZ of up to 32768 rows
+    float* part = nullptr;  // the flat gradient of each part of the rows
     float* grad = nullptr;  // flat gradient [NPARAM]: W[0], b[0], W[1], ...
     float *gW[NL] = {}, *gb[NL] = {};  // its parts
     float* loss_rows = nullptr;
@@ -52,10 +53,11 @@ void mlp_free(Mlp& net);
 hipError_t work_alloc(Work& w, int cap);
 void work_free(Work& w);
 void refresh_bf16(Mlp& net, hipStream_t s);
-void to_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t s);
 // Gradients of the mean-squared loss over the NOUT outputs for one batch (M
-// multiple of 16, at most w.cap) into w.grad; per-row losses land in w.loss_rows.
-void mlp_grad(const Mlp& net, const uint16_t* X, const float* T, int M, Work& w, hipStream_t s);
+// multiple of 16, at most w.cap; X [M][16] in BF16, or in FP32 and rounded to it)
+// into w.grad; per-row losses land in w.loss_rows.
+template <typename XT>
+void mlp_grad(const Mlp& net, const XT* X, const float* T, int M, Work& w, hipStream_t s);
 // One Adam step with the gradients in w; the bias corrections of the step are
 // c12[2 *it], c12[2 *it + 1] (device), filled by adam_corrections (host) for
 // steps first_step .. first_step + iters - 1 (first_step >= 1).

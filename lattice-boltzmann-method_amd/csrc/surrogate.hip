@@ -16,86 +16,39 @@
 namespace lbm {
 namespace sur {
 
-// ------------------------------------------------------- gradient kernel
-// Forward pass, loss and all gradients of the batch in one pass over its rows:
-// a block takes GROWS rows at a time through the four layers and back and keeps
-// its weight gradients in registers.  One wavefront per 16 neurons of the
-// 128-wide layers: with Z^T = W H^T (A operand the weights, i = neuron; B
-// operand the batch rows) the pre-activations a wavefront makes going forward
-// are in its own registers, in place, when the backward pass wants gelu' of
-// them.  Activations and dZ pass between wavefronts as BF16 in LDS, by row for
-// the next layer's product and transposed for the weight gradients, whose
-// reduction index is the row; both strides spread 16 rows of 16 bytes over all
-// banks.  Weights are read where they are used (72 KiB from L2).
-// Bound by the chain of eight phases between barriers.  With a pass per layer
-// and operand (forward, transposes, partial products, their sums, bias sums:
-// 33 launches) a caller's gradient of 4096 rows took 395 us, host copies
-// included, and takes 127.
-constexpr int GWAVES = 8, GROWS = 64, GTILES = GROWS / 16, GSTEPS = GROWS / 32;
-constexpr int GRAD_BLOCKS = 256;       // one per CU: more rows go round
-constexpr int HSTRIDE = 128 + 8, TSTRIDE = GROWS + 8, DSTRIDE = 16 + 8;
-static_assert(GWAVES * 16 == 128, "one wavefront per 16 neurons");
+// ------------------------------------------------------ gradient kernels
+// Forward pass, loss and all gradients of a batch in three launches of small
+// blocks with few registers and little LDS:
+//   k_grad_rows     16 rows a block through the four layers and back, with the
+//                   transposed products Z^T = W H^T of the in-step network;
+//                   activations and dZ leave transposed, as the operands of
+//   k_grad_weights  the weight and bias gradients of a part of the rows, and
+//   k_grad_sum      their sum.
+// Training also runs beside the steps, whose kernels fill the CUs: a block
+// starts only where its registers, wavefronts and LDS fall free at once.  One
+// kernel of 64 rows a block (eight wavefronts of 236 registers, 132 KB of LDS: a
+// whole CU) took 21 us for 4096 rows by itself, but beside the steps it waited
+// for the end of nearly every step kernel: 100 iterations beside 256x128x128
+// FP32 steps took 150 ms or 21 steps.  A block of k_grad_rows takes the place of
+// one block of a collide kernel (124 registers, a wavefront per SIMD, 12 KB): 25
+// ms or 3 steps.  By themselves: k_grad_rows 13 us, bound by its chain of six
+// exchanges between the wavefronts and, from 16384 rows (28 us), by reading the
+// weights per 16 rows; k_grad_weights 10 us, bound by its loads; the sum 3.  A
+// caller's gradient of 4096 rows takes 125 us, host copies included (130 as one
+// kernel), of 16384 rows 198 (206), of 262144 rows 1900 (1500).
+constexpr int GT_H = 0, GT_D = 24, GT_X = 48, GT_D3 = 49, GTILES = 50;  // tiles of a group of 16 rows
+constexpr int GCHUNK = 32768;       // rows whose tiles are held at once (52 MB)
+constexpr int GPART = 8;            // groups (128 rows) whose operands a wavefront holds at once
+constexpr int GPARTS = 64;          // parts of a chunk at most: more groups go round
+// strips of up to four tiles: 16 of each 128x128 layer, 8 of the first, 2 of the last
+constexpr int GSTRIPS = 42;
 
 // Offsets of W[L] and b[L] in the flat gradient.
 constexpr int grad_w(int L) { return frag_offset(L) + bias_offset(L); }
 constexpr int grad_b(int L) { return grad_w(L) + DIMS[L] * DIMS[L + 1]; }
 static_assert(grad_b(NL - 1) + DIMS[NL] == NPARAM, "flat gradient");
 
-// Four neurons n0 + 0..3 of row r, by row and transposed.
-__device__ __forceinline__ void put_rows(uint16_t* h, int r, int n0, const v4s x)
-{
-    uint2 u;
-    __builtin_memcpy(&u, &x, 8);
-    *reinterpret_cast<uint2*>(h + r * HSTRIDE + n0) = u;
-}
-__device__ __forceinline__ void put_cols(uint16_t* hT, int r, int n0, const v4s x)
-{
-#pragma unroll
-    for (int q = 0; q < 4; ++q) hT[(n0 + q) * TSTRIDE + r] = (uint16_t)x[q];
-}
-// acc += A[16 a0 + ..][rows] B[16 b0 + ..][rows]^T over the block's rows
-__device__ __forceinline__ v4f row_products(const v8bf a[GSTEPS], const uint16_t* bT, int b0, v4f acc)
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int s = 0; s < GSTEPS; ++s)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            a[s], load_frag8(bT + (16 * b0 + (lane & 15)) * TSTRIDE + 32 * s + 8 * (lane >> 4)), acc, 0, 0, 0);
-    return acc;
-}
-__device__ __forceinline__ void row_operand(const uint16_t* aT, int a0, v8bf a[GSTEPS])
-{
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int s = 0; s < GSTEPS; ++s)
-        a[s] = load_frag8(aT + (16 * a0 + (lane & 15)) * TSTRIDE + 32 * s + 8 * (lane >> 4));
-}
-// sum over the block's rows of A: the product with ones
-__device__ __forceinline__ v4f row_sums(const v8bf a[GSTEPS], v4f acc)
-{
-    v8bf one;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) one[e] = (__bf16)1.0f;
-#pragma unroll
-    for (int s = 0; s < GSTEPS; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s], one, acc, 0, 0, 0);
-    return acc;
-}
-// out[bt] = W[16 w0 + ..][0..128) h[row][0..128)^T for the block's row tiles
-__device__ __forceinline__ void product128(const uint16_t* W, int w0, const uint16_t* h, v4f out[GTILES])
-{
-    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-    v8bf a[KSTEPS];
-#pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) a[s] = load_frag8(W + (16 * w0 + j) * 128 + 32 * s + 8 * g);
-#pragma unroll
-    for (int bt = 0; bt < GTILES; ++bt) {
-        out[bt] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s)
-            out[bt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                a[s], load_frag8(h + (16 * bt + j) * HSTRIDE + 32 * s + 8 * g), out[bt], 0, 0, 0);
-    }
-}
+// BF16 of a D fragment: the B operand of the next product.
 __device__ __forceinline__ v4s bf_frag(const v4f z)
 {
     v4s r;
@@ -103,165 +56,252 @@ __device__ __forceinline__ v4s bf_frag(const v4f z)
     for (int q = 0; q < 4; ++q) r[q] = (short)f2bf(z[q]);
     return r;
 }
-
-// grid: at most GRAD_BLOCKS blocks of 64 GWAVES threads, M a multiple of 16;
-// part [gridDim.x][NPARAM] receives each block's share of the flat gradient,
-// loss_rows [M] the rows' squared errors.  dZ of the output layer is that of
-// the mean-squared loss over NOUT outputs, 2 (z - t) / (M NOUT), and 0 for
-// padded outputs and for rows past M.
-__global__ __launch_bounds__(64 * GWAVES) void k_grad(Mlp net, const uint16_t* X, const float* T, int M, float* part,
-                                                      float* loss_rows)
+// N tiles from D order (lane: row lane % 16, neurons 4 (lane / 16) + 0..3) to
+// operand order with the row as the reduction index (lane: neuron lane % 16,
+// rows 4 (lane / 16) + 0..3), through the wavefront's own LDS, to `to`.  A
+// wavefront's LDS operations complete in order; the fences keep the compiler to
+// it.
+template <int N>
+__device__ __forceinline__ void put_transposed(uint16_t* lds, const v4s x[N], uint16_t* to)
 {
-    __shared__ __align__(16) uint16_t h[2][GROWS * HSTRIDE];   // by row: activations, then dZ
-    __shared__ __align__(16) uint16_t hT[3][128 * TSTRIDE];    // transposed activations
-    __shared__ __align__(16) uint16_t dT[2][128 * TSTRIDE];    // transposed dZ
-    __shared__ __align__(16) uint16_t xT[16 * TSTRIDE], d3T[16 * TSTRIDE], d3[GROWS * DSTRIDE];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
-    const int n0 = 16 * w + 4 * g;  // the neurons of this lane's D fragments
-    const v4f zero = {0.f, 0.f, 0.f, 0.f};
-    v4f g0 = zero, g1[8], g2[8], g3 = zero, s0 = zero, s1 = zero, s2 = zero, s3 = zero;
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int t = 0; t < 8; ++t) g1[t] = g2[t] = zero;
-    for (int r0 = blockIdx.x * GROWS; r0 < M; r0 += gridDim.x * GROWS) {
-        v4f z0[GTILES], z1[GTILES], z2[GTILES], acc[GTILES];
-        v8bf a[GSTEPS];
-        {  // ---- layer 0, K = 16
-            const v4s wf = load_frag(net.Wb[0] + (16 * w + j) * 16 + 4 * g);
-            const v4f b = bias_frag(net.b[0], 16 * w, lane);
+    for (int t = 0; t < N; ++t)
 #pragma unroll
-            for (int bt = 0; bt < GTILES; ++bt) {
-                const int r = 16 * bt + j;
-                v4s x = {0, 0, 0, 0};
-                if (r0 + r < M) x = load_frag(X + (size_t)(r0 + r) * 16 + 4 * g);
-                if (w == bt) put_cols(xT, r, 4 * g, x);
-                z0[bt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wf, x, zero, 0, 0, 0) + b;
-                const v4s hf = act_frag(z0[bt]);
-                put_rows(h[0], r, n0, hf);
-                put_cols(hT[0], r, n0, hf);
-            }
-        }
-        __syncthreads();
-        // ---- layers 1 and 2
-        auto hidden = [&](int L, const uint16_t* from, uint16_t* to, uint16_t* toT, v4f z[GTILES]) {
-            product128(net.Wb[L], w, from, z);
-            const v4f b = bias_frag(net.b[L], 16 * w, lane);
+        for (int q = 0; q < 4; ++q) lds[t * 256 + (4 * g + q) * 16 + j] = (uint16_t)x[t][q];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-            for (int bt = 0; bt < GTILES; ++bt) {
-                z[bt] += b;
-                const v4s hf = act_frag(z[bt]);
-                put_rows(to, 16 * bt + j, n0, hf);
-                put_cols(toT, 16 * bt + j, n0, hf);
-            }
-        };
-        hidden(1, h[0], h[1], hT[1], z1);
-        __syncthreads();
-        hidden(2, h[1], h[0], hT[2], z2);
-        __syncthreads();
-        // ---- output layer and loss: row tile w
-        if (w < GTILES) {
-            const int r = 16 * w + j, row = r0 + r;
-            v4f z = zero;
+    for (int t = 0; t < N; ++t)
+        *reinterpret_cast<uint2*>(to + t * 256 + lane * 4) =
+            *reinterpret_cast<const uint2*>(lds + t * 256 + j * 16 + 4 * g);
+}
+// The A operands of the two output tiles t0, t0 + 1 of a 128-deep product,
+// forward from the weights in fragment order, backward from W^T by row, and
+// the product with the activations (or dZ) of a layer.
+struct Weights2 {
+    v8bf a[2][KSTEPS];
+};
+__device__ __forceinline__ Weights2 forward_weights(const uint16_t* Wl, int t0)
+{
+    const int lane = threadIdx.x & 63;
+    Weights2 w;
 #pragma unroll
-            for (int s = 0; s < KSTEPS; ++s)
-                z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load_frag8(net.Wb[3] + j * 128 + 32 * s + 8 * g),
-                                                           load_frag8(h[0] + r * HSTRIDE + 32 * s + 8 * g), z, 0, 0, 0);
-            z += bias_frag(net.b[3], 0, lane);
-            v4f dz = zero;
-            float sum = 0.f;
-            if (row < M) {
-                const v4f t = *reinterpret_cast<const v4f*>(T + (size_t)row * 16 + 4 * g);
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (4 * g + q < NOUT) {
-                        const float d = z[q] - t[q];
-                        sum += d * d;
-                        dz[q] = 2.f * d / (float)(M * NOUT);
-                    }
-            }
-            sum += __shfl_xor(sum, 16);
-            sum += __shfl_xor(sum, 32);
-            if (g == 0 && row < M) loss_rows[row] = sum;
-            const v4s df = bf_frag(dz);
-            uint2 u;
-            __builtin_memcpy(&u, &df, 8);
-            *reinterpret_cast<uint2*>(d3 + r * DSTRIDE + 4 * g) = u;
-            put_cols(d3T, r, 4 * g, df);
-        }
-        __syncthreads();
-        // ---- back through the output layer; its weight gradient
-        {
-            const v4s wf = load_frag(net.WbT[3] + (16 * w + j) * 16 + 4 * g);
+        for (int s = 0; s < KSTEPS; ++s) w.a[t][s] = load_frag8(Wl + (((t0 + t) * KSTEPS + s) * 64 + lane) * 8);
+    return w;
+}
+__device__ __forceinline__ Weights2 backward_weights(const uint16_t* WT, int t0)
+{
+    const int lane = threadIdx.x & 63;
+    Weights2 w;
 #pragma unroll
-            for (int bt = 0; bt < GTILES; ++bt) {
-                const int r = 16 * bt + j;
-                v4f d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(wf, load_frag(d3 + r * DSTRIDE + 4 * g), zero, 0, 0, 0);
+    for (int t = 0; t < 2; ++t) {
+        const uint16_t* row = WT + (16 * (t0 + t) + (lane & 15)) * 128 + 4 * (lane >> 4);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) d[q] *= gelu_grad(z2[bt][q]);
-                const v4s df = bf_frag(d);
-                put_rows(h[1], r, n0, df);
-                put_cols(dT[0], r, n0, df);
-            }
-            row_operand(d3T, 0, a);
-            g3 = row_products(a, hT[2], w, g3);
-            s3 = row_sums(a, s3);
-        }
-        __syncthreads();
-        // ---- layer 2
-        product128(net.WbT[2], w, h[1], acc);
-#pragma unroll
-        for (int bt = 0; bt < GTILES; ++bt) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[bt][q] *= gelu_grad(z1[bt][q]);
-            const v4s df = bf_frag(acc[bt]);
-            put_rows(h[0], 16 * bt + j, n0, df);
-            put_cols(dT[1], 16 * bt + j, n0, df);
-        }
-        row_operand(dT[0], w, a);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) g2[t] = row_products(a, hT[1], t, g2[t]);
-        s2 = row_sums(a, s2);
-        __syncthreads();
-        // ---- layer 1
-        product128(net.WbT[1], w, h[0], acc);
-#pragma unroll
-        for (int bt = 0; bt < GTILES; ++bt) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[bt][q] *= gelu_grad(z0[bt][q]);
-            put_cols(dT[0], 16 * bt + j, n0, bf_frag(acc[bt]));
-        }
-        row_operand(dT[1], w, a);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) g1[t] = row_products(a, hT[0], t, g1[t]);
-        s1 = row_sums(a, s1);
-        __syncthreads();
-        // ---- layer 0
-        row_operand(dT[0], w, a);
-        g0 = row_products(a, xT, 0, g0);
-        s0 = row_sums(a, s0);
-        __syncthreads();
+        for (int s = 0; s < KSTEPS; ++s) w.a[t][s] = pair_frag(load_frag(row + 32 * s), load_frag(row + 32 * s + 16));
     }
-    // ---- the block's share, in the flat order
-    float* out = part + (size_t)blockIdx.x * NPARAM;
+    return w;
+}
+__device__ __forceinline__ v4f product128(const v8bf w[KSTEPS], const v4s h[8])
+{
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        out[grad_w(0) + (n0 + q) * 16 + j] = g0[q];
-        out[grad_w(3) + (4 * g + q) * 128 + 16 * w + j] = g3[q];
+    for (int s = 0; s < KSTEPS; ++s)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s], pair_frag(h[2 * s], h[2 * s + 1]), acc, 0, 0, 0);
+    return acc;
+}
+
+// Block b: rows row0 + 16 b + 0..15 (M a multiple of 16, so every row is one of
+// the batch), wavefront w neurons 32 w + 0..31 of each 128-wide layer; the
+// output layer is evaluated by every wavefront.  X holds BF16 features, or binary32
+// ones that are rounded here.  loss_rows [M] receives the rows' squared errors.
+// dZ of the output layer is that of the mean-squared loss over NOUT outputs,
+// 2 (z - t) / (M NOUT), and 0 for padded outputs.  Each layer's weights are on
+// their way while the layer before it is evaluated and shared.
+template <typename XT>
+__global__ __launch_bounds__(256) void k_grad_rows(Mlp net, const XT* X, const float* T, int M, int row0, uint16_t* tiles,
+                                                   float* loss_rows)
+{
+    __shared__ __align__(16) uint16_t turn[4][2 * 256];
+    __shared__ __align__(16) uint16_t frags[2][8 * 256];  // a layer's activations or dZ, from all wavefronts
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
+    const int row = row0 + blockIdx.x * 16 + j;
+    uint16_t* const out = tiles + (size_t)blockIdx.x * (GTILES * 256);
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    v4f z0[2], z1[2], z2[2];
+    v4s mine[2], all[8];
+    // the wavefront's two tiles to the others (buffer p) and, transposed, to memory
+    auto share = [&](int p, int tile) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            out[grad_w(1) + (n0 + q) * 128 + 16 * t + j] = g1[t][q];
-            out[grad_w(2) + (n0 + q) * 128 + 16 * t + j] = g2[t][q];
+        for (int t = 0; t < 2; ++t) {
+            uint2 u;
+            __builtin_memcpy(&u, &mine[t], 8);
+            *reinterpret_cast<uint2*>(frags[p] + (2 * w + t) * 256 + lane * 4) = u;
         }
-        if (j == 0) {
-            out[grad_b(0) + n0 + q] = s0[q];
-            out[grad_b(1) + n0 + q] = s1[q];
-            out[grad_b(2) + n0 + q] = s2[q];
-            if (w == 0) out[grad_b(3) + 4 * g + q] = s3[q];
+        put_transposed<2>(turn[w], mine, out + (tile + 2 * w) * 256);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 8; ++t) all[t] = load_frag(frags[p] + t * 256 + lane * 4);
+    };
+    // ---- forward
+    const int n0 = 32 * w;
+    Weights2 wt = forward_weights(net.Wf + frag_offset(1), 2 * w);
+    v4s x[1];
+    if constexpr (sizeof(XT) == 2) x[0] = load_frag(X + (size_t)row * 16 + 4 * g);
+    else x[0] = bf_frag(*reinterpret_cast<const v4f*>(X + (size_t)row * 16 + 4 * g));
+    if (w == 0) put_transposed<1>(turn[0], x, out + GT_X * 256);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        z0[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(load_frag(net.Wb[0] + (n0 + 16 * t + j) * 16 + 4 * g), x[0],
+                                                         zero, 0, 0, 0) +
+                bias_frag(net.b[0], n0 + 16 * t, lane);
+        mine[t] = act_frag(z0[t]);
+    }
+    share(0, GT_H);
+    Weights2 nx = forward_weights(net.Wf + frag_offset(2), 2 * w);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        z1[t] = product128(wt.a[t], all) + bias_frag(net.b[1], n0 + 16 * t, lane);
+        mine[t] = act_frag(z1[t]);
+    }
+    share(1, GT_H + 8);
+#pragma unroll
+    for (int s = 0; s < KSTEPS; ++s) wt.a[0][s] = load_frag8(net.Wf + frag_offset(3) + (s * 64 + lane) * 8);
+    const v4f target = *reinterpret_cast<const v4f*>(T + (size_t)row * 16 + 4 * g);
+    const v4s w3[2] = {load_frag(net.WbT[3] + (n0 + j) * 16 + 4 * g), load_frag(net.WbT[3] + (n0 + 16 + j) * 16 + 4 * g)};
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        z2[t] = product128(nx.a[t], all) + bias_frag(net.b[2], n0 + 16 * t, lane);
+        mine[t] = act_frag(z2[t]);
+    }
+    share(0, GT_H + 16);
+    nx = backward_weights(net.WbT[2], 2 * w);
+    const v4f z3 = product128(wt.a[0], all) + bias_frag(net.b[3], 0, lane);
+    // ---- loss and its gradient
+    v4f dz = zero;
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (4 * g + q < NOUT) {
+            const float d = z3[q] - target[q];
+            sum += d * d;
+            dz[q] = 2.f * d / (float)(M * NOUT);
         }
+    const v4s d3[1] = {bf_frag(dz)};
+    if (w == 0) {
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if (g == 0) loss_rows[row] = sum;
+        put_transposed<1>(turn[0], d3, out + GT_D3 * 256);
+    }
+    // ---- backward
+    auto through_gelu = [&](v4f d, const v4f z) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[q] *= gelu_grad(z[q]);
+        return bf_frag(d);
+    };
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+        mine[t] = through_gelu(__builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w3[t], d3[0], zero, 0, 0, 0), z2[t]);
+    share(1, GT_D + 16);
+    wt = backward_weights(net.WbT[1], 2 * w);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) mine[t] = through_gelu(product128(nx.a[t], all), z1[t]);
+    share(0, GT_D + 8);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) mine[t] = through_gelu(product128(wt.a[t], all), z0[t]);
+    put_transposed<2>(turn[w], mine, out + (GT_D + 2 * w) * 256);
+}
+
+// NB 16x16 tiles of a weight gradient over groups [first, last), two groups (32
+// rows) to an instruction, operand tile ta against tb + 0..NB-1, and the sums
+// over the rows of ta (its product with ones).
+template <int NB>
+__device__ __forceinline__ void weight_strip(const uint16_t* tiles, int ta, int tb, int first, int last, v4f acc[NB],
+                                             v4f& sums)
+{
+    const int lane = threadIdx.x & 63;
+    v8bf one;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) one[e] = (__bf16)1.0f;
+    // every load ahead of its use: groups past the last one read the part's
+    // first and count as zero
+    uint2 x[GPART][NB + 1];
+#pragma unroll
+    for (int r = 0; r < GPART; ++r) {
+        const uint16_t* p = tiles + (size_t)(first + r < last ? first + r : first) * (GTILES * 256) + lane * 4;
+        x[r][0] = *reinterpret_cast<const uint2*>(p + ta * 256);
+#pragma unroll
+        for (int t = 0; t < NB; ++t) x[r][1 + t] = *reinterpret_cast<const uint2*>(p + (tb + t) * 256);
+    }
+#pragma unroll
+    for (int r = 0; r < GPART; ++r)
+#pragma unroll
+        for (int t = 0; t <= NB; ++t)
+            if (first + r >= last) x[r][t] = make_uint2(0, 0);
+    auto operand = [](const uint2 lo, const uint2 hi) {
+        const uint2 u[2] = {lo, hi};
+        v8bf o;
+        __builtin_memcpy(&o, u, 16);
+        return o;
+    };
+#pragma unroll
+    for (int r = 0; r < GPART; r += 2) {
+        const v8bf a = operand(x[r][0], x[r + 1][0]);
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, operand(x[r][1 + t], x[r + 1][1 + t]), acc[t], 0, 0, 0);
+        sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, one, sums, 0, 0, 0);
     }
 }
 
-// Sums the blocks' shares in a fixed order: 64 parameters per block of 256, a
-// quarter of the shares per wavefront.
+// grid (GSTRIPS, parts): one wavefront forms a strip of one layer's weight gradient
+// over its part of the groups and, with a neuron tile's first strip, its
+// bias gradient.  part [blockIdx.y][NPARAM] is written, or added to when `more`.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 4))) void
+k_grad_weights(const uint16_t* tiles, int groups, int more, float* part)
+{
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    float* const out = part + (size_t)blockIdx.y * NPARAM;
+    auto put = [&](int i, float v) { out[i] = more ? out[i] + v : v; };
+    // tiles na (neurons) x nb.. (inputs) of layer L
+    auto strip = [&](auto count, int L, int na, int nb, int ta, int tb) {
+        constexpr int NB = decltype(count)::value;
+        v4f acc[NB], sums = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < NB; ++t) acc[t] = sums;
+        for (int first = blockIdx.y * GPART; first < groups; first += gridDim.y * GPART)
+            weight_strip<NB>(tiles, ta, tb, first, min(first + GPART, groups), acc, sums);
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                put(grad_w(L) + (16 * na + 4 * g + q) * DIMS[L] + 16 * (nb + t) + j, acc[t][q]);
+        if (j == 0 && nb == 0) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) put(grad_b(L) + 16 * na + 4 * g + q, sums[q]);
+        }
+    };
+    using One = std::integral_constant<int, 1>;
+    using Four = std::integral_constant<int, 4>;
+    const int id = blockIdx.x;
+    if (id < 32) {
+        const int L = 1 + (id >> 4), na = (id & 15) >> 1, nb = 4 * (id & 1);
+        strip(Four{}, L, na, nb, GT_D + 8 * L + na, GT_H + 8 * (L - 1) + nb);
+    } else if (id < 40) {
+        strip(One{}, 0, id - 32, 0, GT_D + id - 32, GT_X);
+    } else {
+        strip(Four{}, 3, 0, 4 * (id - 40), GT_D3, GT_H + 16 + 4 * (id - 40));
+    }
+}
+
+// Sums the parts in a fixed order: 64 parameters per block of 256, a quarter of
+// the parts per wavefront.
 __global__ __launch_bounds__(256) void k_grad_sum(const float* part, int nblk, float* grad)
 {
     __shared__ float red[4][64];
@@ -297,12 +337,6 @@ __global__ void k_adam(float* w, const float* g, float* m, float* v, int n, floa
         const int r = i / cols, c = i % cols;
         wbT[(size_t)c * rows + r] = f2bf(wi);
     }
-}
-
-__global__ void k_to_bf(const float* in, uint16_t* out, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = f2bf(in[i]);
 }
 
 // W[L] (FP32, [N][K]) into the fragment-ordered BF16 block of layer L: the
@@ -508,7 +542,15 @@ __global__ __launch_bounds__(256) void k_loss_sum(const float* lr, int B, float 
 {
     __shared__ float red[256];
     float s = 0.f;
-    for (int i = threadIdx.x; i < B; i += 256) s += lr[i];
+    int i = threadIdx.x;
+    for (; i + 7 * 256 < B; i += 8 * 256) {  // eight loads on their way, added in order
+        float x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = lr[i + k * 256];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s += x[k];
+    }
+    for (; i < B; i += 256) s += lr[i];
     red[threadIdx.x] = s;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
@@ -523,14 +565,26 @@ void loss_sum(const float* loss_rows, int B, float scale, float* out, hipStream_
     hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(256), 0, s, loss_rows, B, scale, out, idx);
 }
 
-static int grad_blocks(int M) { return cdiv(M, GROWS) < GRAD_BLOCKS ? cdiv(M, GROWS) : GRAD_BLOCKS; }
-
-void mlp_grad(const Mlp& net, const uint16_t* X, const float* T, int M, Work& w, hipStream_t s)
+// parts of the (first) chunk of M rows
+static int grad_parts(int M)
 {
-    const int nblk = grad_blocks(M);
-    hipLaunchKernelGGL(k_grad, dim3(nblk), dim3(64 * GWAVES), 0, s, net, X, T, M, w.part, w.loss_rows);
-    hipLaunchKernelGGL(k_grad_sum, dim3(cdiv(NPARAM, 64)), dim3(256), 0, s, w.part, nblk, w.grad);
+    const int n = cdiv((M < GCHUNK ? M : GCHUNK) / 16, GPART);
+    return n < GPARTS ? n : GPARTS;
 }
+
+template <typename XT>
+void mlp_grad(const Mlp& net, const XT* X, const float* T, int M, Work& w, hipStream_t s)
+{
+    for (int row0 = 0; row0 < M; row0 += GCHUNK) {
+        const int groups = (M - row0 < GCHUNK ? M - row0 : GCHUNK) / 16;
+        hipLaunchKernelGGL(k_grad_rows<XT>, dim3(groups), dim3(256), 0, s, net, X, T, M, row0, w.tiles, w.loss_rows);
+        hipLaunchKernelGGL(k_grad_weights, dim3(GSTRIPS, grad_parts(M - row0)), dim3(64), 0, s, w.tiles, groups,
+                           row0 > 0 ? 1 : 0, w.part);
+    }
+    hipLaunchKernelGGL(k_grad_sum, dim3(cdiv(NPARAM, 64)), dim3(256), 0, s, w.part, grad_parts(M), w.grad);
+}
+template void mlp_grad<uint16_t>(const Mlp&, const uint16_t*, const float*, int, Work&, hipStream_t);
+template void mlp_grad<float>(const Mlp&, const float*, const float*, int, Work&, hipStream_t);
 
 void adam_corrections(int first_step, int iters, float* c12)
 {
@@ -554,11 +608,6 @@ void mlp_adam(Mlp& net, Work& w, float lr, const float* c12, const int* it, hipS
         hipLaunchKernelGGL(k_to_frag, dim3(cdiv(n, 256)), dim3(256), 0, s, net.W[L], DIMS[L + 1], DIMS[L],
                            net.Wf + frag_offset(L));
     }
-}
-
-void to_bf16(const float* in, uint16_t* out, int64_t n, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_to_bf, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, out, n);
 }
 
 void refresh_bf16(Mlp& net, hipStream_t s)
@@ -673,7 +722,9 @@ void mlp_free(Mlp& net)
 // (cap is set once everything is there: a caller asks it whether to allocate)
 hipError_t work_alloc(Work& w, int cap)
 {
-    hipError_t e = hipMalloc((void**)&w.part, sizeof(float) * NPARAM * (size_t)grad_blocks(cap));
+    const size_t rows = (size_t)(cap < GCHUNK ? cap : GCHUNK);
+    hipError_t e = hipMalloc((void**)&w.tiles, sizeof(uint16_t) * 16 * GTILES * rows);
+    if (e == hipSuccess) e = hipMalloc((void**)&w.part, sizeof(float) * NPARAM * (size_t)grad_parts(cap));
     if (e == hipSuccess) e = hipMalloc((void**)&w.grad, sizeof(float) * NPARAM);
     if (e == hipSuccess) e = hipMalloc((void**)&w.loss_rows, sizeof(float) * (size_t)cap);
     if (e == hipSuccess) e = hipMalloc((void**)&w.xf, sizeof(float) * 16 * (size_t)cap);
@@ -691,7 +742,7 @@ hipError_t work_alloc(Work& w, int cap)
 
 void work_free(Work& w)
 {
-    void* ps[] = {w.part, w.grad, w.loss_rows, w.xf};
+    void* ps[] = {w.tiles, w.part, w.grad, w.loss_rows, w.xf};
     for (void* p : ps)
         if (p) (void)hipFree(p);
     w = Work{};

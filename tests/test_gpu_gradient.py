@@ -1,11 +1,14 @@
-"""The network's gradient kernel at the edges of its row groups against the
+"""The network's gradient kernels at the edges of their row groups against the
 oracle, through the C ABI.
 
-A block takes 64 rows at a time (four tiles of 16) and at most 256 blocks share
-a batch, so: one tile, a partly filled group, a full one, one row tile more, and
-a second round of the first blocks.  Both sides round activations and dZ to
-BF16 at the same places, so they differ by FP32 sums and by the roundings those
-flip: 1e-4 of the loss, 1e-2 of a layer's gradient norm, at any row count.
+A block of the rows' kernel takes 16 rows; a wavefront of the weights' kernel
+takes parts of 8 such groups (128 rows), two groups to an instruction, at most 64
+parts at once (8192 rows), and batches go in chunks of 32768 rows.  So: one
+group, an odd number of groups, a full pair, a part and one group more, a second
+round of the first parts, and a second chunk.  Both sides round activations
+and dZ to BF16 at the same places, so they differ by FP32 sums and by the
+roundings those flip: 1e-4 of the loss, 1e-2 of a layer's gradient norm, at any
+row count.
 """
 import numpy as np
 import pytest
@@ -16,7 +19,7 @@ from test_gpu_surrogate import box, lattice, scaled_params
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows", [16, 48, 64, 80, 16384 + 16])
+@pytest.mark.parametrize("rows", [16, 48, 64, 80, 16384 + 16, 128 + 16, 8192 + 16, 32768 + 16])
 def test_gradient_matches_oracle_at_row_group_edges(rows):
     lat = lattice(box())
     params = scaled_params(9, 1.2)
