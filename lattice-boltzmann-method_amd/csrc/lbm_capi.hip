@@ -1917,9 +1917,6 @@ int collide_overlapped(lbm_ctx* c)
         if (ee == hipSuccess) ee = hipStreamWaitEvent(es, c->ev_trans, 0);
     }
     if (!rc) rc = run_mc_on(c, es, McKernel::Collide, "mc_collide_mixture", 0, 1);
-    const bool energy = !rc && (push || inplace(c));
-    if (energy) rc = run_mc_on(c, es, McKernel::StreamEnergy, "mc_stream_energy", 1, 0);
-    if (ee == hipSuccess && es != c->stream) ee = hipEventRecord(c->ev_edone, es);
     HIP_TRY(c, ec);
     HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_cdone, 0));
     if (!rc && inplace(c)) {
@@ -1930,6 +1927,11 @@ int collide_overlapped(lbm_ctx* c)
     } else if (!rc) {
         rc = run_mc(c, McKernel::CollideSpecies, "mc_collide_species", 0, 1);
     }
+    // (queued last: a step whose species collide is refused, for instance for
+    // want of memory, leaves the energy populations where lbm_collide does)
+    const bool energy = !rc && (push || inplace(c));
+    if (energy) rc = run_mc_on(c, es, McKernel::StreamEnergy, "mc_stream_energy", 1, 0);
+    if (ee == hipSuccess && es != c->stream) ee = hipEventRecord(c->ev_edone, es);
     HIP_TRY(c, ee);
     if (es != c->stream) HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_edone, 0));
     c->energy_streamed = energy && !rc;

@@ -10,7 +10,8 @@ follow the energy stream, and two charges on a grid of a few wavefronts.
 import pytest
 
 from lbm_amd import cases
-from lbm_amd.capi import LBM_FP32_SHIFTED, LBM_FP64, LBM_MODE_FUSED, LBM_MODE_INPLACE, LBM_MODE_STRICT
+from lbm_amd.capi import (LBM_FP32_SHIFTED, LBM_FP64, LBM_MODE_FUSED, LBM_MODE_INPLACE, LBM_MODE_STRICT, POP_F, POP_G,
+                          LbmError)
 from mode_compare import assert_same, make, snapshot
 
 pytestmark = pytest.mark.gpu
@@ -45,6 +46,27 @@ def test_overlapped_step_matches_serial_calls(case, mode, precision, reaction):
         ov.step(3)
         ser.step(3)
         assert_same(snapshot(ov, F), snapshot(ser, F), "three steps in one call")
+    finally:
+        ov.close()
+        ser.close()
+
+
+def test_refused_step_leaves_the_energy_populations(monkeypatch):
+    """An in-place step whose species collide is refused (LBM_AMD_LOW_MAX below
+    one species' floor pairs) must leave the populations as the refused serial
+    call does: the energy populations stream only in a step that goes through."""
+    monkeypatch.setenv("LBM_AMD_LOW_MAX", "100")
+    fl = cases.reacting_box(6, 5, 4, T_K=1300.0, amp_T=0.1, amp_u=0.01, X={"O2": 0.3, "N2": 0.7})
+    ov, ser = (make(fl, LBM_MODE_INPLACE, LBM_FP64, False) for _ in range(2))
+    try:
+        before = ov.get_populations(POP_G)
+        with pytest.raises(LbmError, match="SPECIES_MIN"):
+            ov.step(1)
+        with pytest.raises(LbmError, match="SPECIES_MIN"):
+            ser.Collide_Species()
+        assert (ser.get_populations(POP_G) == before).all()
+        assert (ov.get_populations(POP_G) == before).all()
+        assert (ov.get_populations(POP_F) == ser.get_populations(POP_F)).all()
     finally:
         ov.close()
         ser.close()
