@@ -444,6 +444,18 @@ constexpr bool any_plog()
     return false;
 }
 
+// log10 of Troe's broadening factor from log10 of the reduced pressure and of
+// the factor at its centre.  Plain divisions: where the inner divisor passes
+// through zero its quotient is infinite and the factor 1, and through a
+// reciprocal it would be NaN.
+__host__ __device__ inline double troe_log_f(double lPr, double lFc)
+{
+    const double cc = -0.4 - 0.67 * lFc;
+    const double nn = 0.75 - 1.27 * lFc;
+    const double f1 = (lPr + cc) / (nn - 0.14 * (lPr + cc));
+    return lFc / (1.0 + f1 * f1);
+}
+
 // Net molar production rates [kmol/m^3/s] at (T, rho, Y), SI units.
 __host__ __device__ inline void net_production(double T, double rho, const double Y[NS], double wdot[NS])
 {
@@ -487,12 +499,8 @@ __host__ __device__ inline void net_production(double T, double rho, const doubl
                     double Fc = (1.0 - TROE[r][0]) * exp(quot(-T, Divisor{TROE[r][1], 1.0 / TROE[r][1]})) +
                                 TROE[r][0] * exp(quot(-T, Divisor{TROE[r][2], 1.0 / TROE[r][2]}));
                     if (TROE_HAS_T2[r]) Fc += exp(-TROE[r][3] * invT);
-                    const double lFc = log10(Fc);
                     const double lPr = log10(Pr > 1e-300 ? Pr : 1e-300);
-                    const double cc = -0.4 - 0.67 * lFc;
-                    const double nn = 0.75 - 1.27 * lFc;
-                    const double f1 = quot(lPr + cc, nn - 0.14 * (lPr + cc));
-                    kf = quot(kf * Pr, 1.0 + Pr) * exp10(quot(lFc, 1.0 + f1 * f1));
+                    kf = quot(kf * Pr, 1.0 + Pr) * exp10(troe_log_f(lPr, log10(Fc)));
                 } else {  // Lindemann: broadening factor 1
                     kf = quot(kf * Pr, 1.0 + Pr);
                 }
