@@ -53,13 +53,19 @@ __host__ __device__ inline float rcp_r(float x)
 // moment kernels.  Most of their divisors are constants (molar masses) or shared
 // by many quotients (rho, T, a pivot), so a divisor carries its reciprocal
 // and a quotient takes three: the approximate quotient, its exact residual by
-// fused multiply-add and the correction (Markstein 1990).  The result is the
-// correctly rounded quotient (the error before the last rounding is below
-// 2^-51 units in the last place), so it is bit for bit that of `/`, for
-// divisors and quotients in the normal range; an infinite quotient or a zero
-// divisor gives NaN.  Host code divides.
+// fused multiply-add and the correction (Markstein 1990).  With y the correctly
+// rounded 1 / b the result is the correctly rounded quotient, bit for bit that of
+// `/`, for divisors and quotients in the normal range.  (With y the other
+// neighbour of 1 / b it is not for three in ten of the quotients that lie as close
+// to the middle of two numbers as they come.)  The Newton steps of divisor() give
+// the correctly rounded y unless 1 / b lies within 2^-88 of itself of a middle:
+// for a few divisors less than 2^-42 below a power of two, over which a quotient
+// next to a middle may round to the other side (1 over 2 - 2^-52 does).  Tested
+// on the host and on the device.  A zero or infinite divisor and an infinite
+// quotient give NaN, and -0 gives 0: a division that may meet one is written `/`.
+// Host code divides.
 struct Divisor {
-    double b, y;  // the divisor and 1 / b to within 2^-52
+    double b, y;  // the divisor and 1 / b, correctly rounded
 };
 // a / d.b by the residual correction
 __host__ __device__ inline double quotient_fma(double a, const Divisor& d)
@@ -68,7 +74,8 @@ __host__ __device__ inline double quotient_fma(double a, const Divisor& d)
     const double r = __builtin_fma(-q, d.b, a);
     return __builtin_fma(r, d.y, q);
 }
-// 1 / b: the hardware's approximate reciprocal and two Newton steps
+// 1 / b: the hardware's approximate reciprocal (2^-22 or better) and two Newton
+// steps, 2^-88 before the last rounding
 __host__ __device__ inline Divisor divisor(double b)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
