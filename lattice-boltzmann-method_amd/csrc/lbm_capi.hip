@@ -14,6 +14,8 @@
 #include <thread>
 #include <vector>
 
+#include <sched.h>
+
 #include "lbm_amd.h"
 #include "lbm_internal.h"
 #include "lbm_multi.h"
@@ -31,8 +33,11 @@ thread_local std::string g_create_error;
 struct Stage {
     static constexpr int WORKERS = 8, SLOTS = 2 * WORKERS;
     static constexpr size_t CHUNK = (size_t)1 << 20;
-    // below this the copy through the runtime's own staging takes about as long
-    // as starting the threads saves
+    // Smaller copies go through the runtime's own staging: starting the threads
+    // takes 0.15 ms.  Staged and direct, in ms: 3.9 MiB of binary64 0.30 and 0.22,
+    // 7.9 MiB 0.39 and 0.46, 16 MiB 0.58 and 0.95, 32 MiB 1.3 and 3.2; binary32
+    // planes of 9 to 10 MiB 0.5 to 1.6 and 1.0 to 1.8 (the most where the process's
+    // pages are new), of 18.9 MiB 0.74 to 3.0 and 4.0.
     static constexpr size_t LEAST = (size_t)16 << 20;
     char* pinned = nullptr;
     hipEvent_t ev[SLOTS] = {};
@@ -536,13 +541,25 @@ void release(lbm_ctx* c)
     if (c->stream) (void)hipStreamDestroy(c->stream);
 }
 
+// Threads for a staged download.
+int copying_threads()
+{
+    cpu_set_t set;
+    const int cores = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : Stage::WORKERS;
+    return std::max(1, std::min(cores, Stage::WORKERS));
+}
+
 // Downloads `bytes` of device memory in stream order: put(src, offset, len)
 // receives each chunk in pinned host memory, in any order and from several
 // threads, and copies or converts it to its place.  A copy to pageable memory
 // runs at one thread's pace, which faults in the caller's new pages and copies
-// them; eight threads do both while the bus brings the next chunks.  Five
+// them; up to eight threads do both while the bus brings the next chunks.  Five
 // fields of 258^3 values: 73.6 -> 26 ms; nine binary32 planes of 258x130x130,
 // converted on the way: 57.9 -> 5.6 ms.
+// The threads start once the first chunk has arrived: until then one thread
+// waits (256^3 FP32 after 100 steps: 0.28 s of one core, 2.4 s of nine
+// cores' time when they started at once).  There are no more of them than cores
+// that the process may use.
 // False when nothing was staged (a small copy, or no threads or pinned memory to
 // be had): the caller copies by itself.
 template <typename Put>
@@ -562,6 +579,7 @@ bool staged_download(lbm_ctx* c, const void* dev, size_t bytes, Put put, int* rc
         }
     }
     const size_t chunks = (bytes + Stage::CHUNK - 1) / Stage::CHUNK;
+    const int workers = copying_threads();
     std::atomic<size_t> queued{0};            // chunks whose copy and event are on the stream
     std::atomic<int> error{hipSuccess};
     std::atomic<bool> stop{false};
@@ -569,7 +587,7 @@ bool staged_download(lbm_ctx* c, const void* dev, size_t bytes, Put put, int* rc
     for (auto& f : full) f.store(false);
     auto work = [&](int w) {
         (void)hipSetDevice(c->cfg.device);
-        for (size_t k = w; k < chunks; k += Stage::WORKERS) {
+        for (size_t k = w; k < chunks; k += workers) {
             while (queued.load(std::memory_order_acquire) <= k) {
                 if (stop.load()) return;
                 std::this_thread::yield();
@@ -586,34 +604,48 @@ bool staged_download(lbm_ctx* c, const void* dev, size_t bytes, Put put, int* rc
             full[slot].store(false, std::memory_order_release);
         }
     };
+    auto queue = [&](size_t k) {
+        const int slot = (int)(k % Stage::SLOTS);
+        const size_t off = k * Stage::CHUNK;
+        hipError_t e = hipMemcpyAsync(st.pinned + slot * Stage::CHUNK, static_cast<const char*>(dev) + off,
+                                      std::min(Stage::CHUNK, bytes - off), hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipEventRecord(st.ev[slot], c->stream);
+        if (e != hipSuccess) {
+            error.store(e);
+            stop.store(true);
+            return;
+        }
+        full[slot].store(true, std::memory_order_release);
+        queued.store(k + 1, std::memory_order_release);
+    };
+    size_t k = 0;
+    for (; k < chunks && k < Stage::SLOTS && !stop.load(); ++k) queue(k);
+    if (!stop.load()) {
+        const hipError_t e = hipEventSynchronize(st.ev[0]);
+        if (e != hipSuccess) {
+            error.store(e);
+            stop.store(true);
+        }
+    }
     std::thread pool[Stage::WORKERS];
     bool started = true;
     try {
-        for (int w = 0; w < Stage::WORKERS; ++w) pool[w] = std::thread(work, w);
-    } catch (const std::exception&) {  // no thread to be had: nothing is queued yet
+        for (int w = 0; w < workers && !stop.load(); ++w) pool[w] = std::thread(work, w);
+    } catch (const std::exception&) {  // no thread to be had
         started = false;
         stop.store(true);
     }
-    if (started)
-        for (size_t k = 0; k < chunks && !stop.load(); ++k) {
-            const int slot = (int)(k % Stage::SLOTS);
-            while (full[slot].load(std::memory_order_acquire) && !stop.load()) std::this_thread::yield();
-            if (stop.load()) break;
-            const size_t off = k * Stage::CHUNK;
-            hipError_t e = hipMemcpyAsync(st.pinned + slot * Stage::CHUNK, static_cast<const char*>(dev) + off,
-                                          std::min(Stage::CHUNK, bytes - off), hipMemcpyDeviceToHost, c->stream);
-            if (e == hipSuccess) e = hipEventRecord(st.ev[slot], c->stream);
-            if (e != hipSuccess) {
-                error.store(e);
-                stop.store(true);
-                break;
-            }
-            full[slot].store(true, std::memory_order_release);
-            queued.store(k + 1, std::memory_order_release);
-        }
+    for (; k < chunks && !stop.load(); ++k) {
+        while (full[k % Stage::SLOTS].load(std::memory_order_acquire) && !stop.load()) std::this_thread::yield();
+        if (!stop.load()) queue(k);
+    }
     for (auto& t : pool)
         if (t.joinable()) t.join();
-    if (!started) return false;
+    if (!started) {
+        const hipError_t e = hipStreamSynchronize(c->stream);  // no copy may still write the slots
+        if (e != hipSuccess) *rc = fail(c, LBM_E_HIP, std::string("download: ") + hipGetErrorString(e));
+        return e != hipSuccess;
+    }
     if (error.load() != hipSuccess) {
         (void)hipStreamSynchronize(c->stream);  // no copy may still write the slots
         *rc = fail(c, LBM_E_HIP, std::string("download: ") + hipGetErrorString((hipError_t)error.load()));

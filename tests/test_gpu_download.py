@@ -5,6 +5,7 @@ per cell and read back whole: every field (binary64), species planes and
 populations (binary32 storage with its per-plane shifts), a length that is
 no multiple of the chunk, twice over and from two threads with a context each."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -73,3 +74,30 @@ def test_two_threads_download_at_once():
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not errs
+
+
+def test_waiting_for_queued_steps_takes_one_thread():
+    """A field read after queued steps: the wait for them is one thread's, the copying
+    threads start after it.  So the read takes the processor time of the same read
+    without queued steps and, at most, the wait's twice over (the waiting thread may
+    spin, and the runtime has a thread of its own); eight waiting threads take more."""
+    lat = Lattice(256, 256, 256, 0.1, precision=LBM_FP32_SHIFTED)
+    fl = cases.default_fields(256, 256, 256)
+    cases.periodic_ghosts(fl)
+    fl["p"][...], fl["T"][...] = 1.0 / 3.0, 1.0
+    lat.load_case(fl)
+    lat.Init()
+
+    def read():
+        wall, cpu = time.perf_counter(), time.process_time()
+        lat.get_field("T")
+        return time.perf_counter() - wall, time.process_time() - cpu
+
+    lat.step(3)
+    lat.get_field("T")
+    lat.sync()
+    _, idle = read()
+    lat.step(80)
+    wall, cpu = read()
+    lat.close()
+    assert cpu - idle < 2 * wall, (wall, cpu, idle)
