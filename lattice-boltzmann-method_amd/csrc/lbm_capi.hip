@@ -20,6 +20,7 @@
 #include "lbm_internal.h"
 #include "lbm_multi.h"
 #include "surrogate.h"
+#include "sweep_lists.h"
 
 using namespace lbm;
 
@@ -1063,19 +1064,7 @@ int lbm_set_types(lbm_ctx* c, const uint8_t* types)
         // off their entries and follow the other sweep's results there: the two
         // run at once only with five cells between their entries.
         constexpr int FAR = 5;
-        c->tms_apart = true;
-        std::vector<uint8_t> near(tcell.empty() || icell.empty() ? 0 : (size_t)d.n, 0);
-        if (!near.empty()) {
-            for (int t : tcell) near[t] = 1;
-            for (int t : icell) {
-                const int i = t / (d.ny * d.nz), j = t / d.nz % d.ny, k = t % d.nz;
-                for (int a = std::max(i - FAR, 0); a <= std::min(i + FAR, d.nx - 1); ++a)
-                    for (int b = std::max(j - FAR, 0); b <= std::min(j + FAR, d.ny - 1); ++b)
-                        for (int e = std::max(k - FAR, 0); e <= std::min(k + FAR, d.nz - 1); ++e)
-                            if (near[((int64_t)a * d.ny + b) * d.nz + e]) c->tms_apart = false;
-                if (!c->tms_apart) break;
-            }
-        }
+        c->tms_apart = sweeps_apart(tcell, icell, d.ny, d.nz, FAR);
         tcell.insert(tcell.end(), icell.begin(), icell.end());
         tdir.insert(tdir.end(), idir.begin(), idir.end());
         if (!tcell.empty()) {
