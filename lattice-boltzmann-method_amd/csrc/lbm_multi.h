@@ -83,8 +83,7 @@ constexpr unsigned CHEM_AUDIT = 0x80000000u;
 // species sets in fo from the streamed f.
 // SpeciesTransport runs first in Collide_Species (per cell: omega_a and the
 // Maxwell-Stefan friction), then CollideSpecies or CollideSpeciesPush.
-// ChemistryBeside is Chemistry launched to share the CUs with the kernels of
-// another stream.
+// ChemistryBeside is Chemistry launched beside the kernels of other streams.
 enum class McKernel { Init, Chemistry, ChemistryBeside, SpeciesTransport, CollideSpecies, Collide, Stream, Moments, CollideSpeciesPush,
                       StreamEnergy, SideFill, Unstream };
 

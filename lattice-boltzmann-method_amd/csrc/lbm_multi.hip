@@ -2634,6 +2634,30 @@ constexpr bool kernels_built()
     return sizeof(P) == 8 || NS <= 16;
 }
 
+static int cu_count()
+{
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    return cus;
+}
+
+// Whether the chemistry beside the other streams is held to one block per CU (by
+// claiming more than half its LDS), a wavefront per SIMD, so that their kernels
+// find registers.  Without that it takes all the registers it can get, which is
+// the faster step but for two kinds of grid: binary32 storage in place, and grids
+// of no more than two blocks per CU, whose blocks it spreads.  Steps held and
+// not, in us, with 9 and 6 species: in place FP32 131x97x75 1581 and 1616, 1165
+// and 1187; 160x128x128 4202 and 4351, 3034 and 3098; 2048x4x4 flame FP64 314 and
+// 321; 40x48x40 FP64 267 and 269, 174 and 174.  On the other side 64^3 FP32 462 and
+// 440, 391 and 360; 64^3 FP64 778 and 775, 586 and 558; 96x80x64 strict 1917 and
+// 1900, 1392 and 1317; 160x128x128 6887 and 6818, 4796 and 4771.
+template <typename P>
+static bool chemistry_alone(const MultiView<P>& v)
+{
+    const bool one_buffer = v.f == v.fo;  // in place
+    return (sizeof(P) == 4 && one_buffer) || v.d.n <= (int64_t)2 * BLOCK * cu_count();
+}
+
 template <typename P>
 void launch_mc(McKernel k, const MultiView<P>& v, hipStream_t s)
 {
@@ -2644,14 +2668,7 @@ void launch_mc(McKernel k, const MultiView<P>& v, hipStream_t s)
         case McKernel::Init: hipLaunchKernelGGL(k_mc_init<P>, grid1(v.d.n), dim3(BLOCK), 0, s, v); break;
         case McKernel::Chemistry: hipLaunchKernelGGL(k_mc_chemistry<P>, grid1(v.d.n), dim3(BLOCK), 0, s, v); break;
         case McKernel::ChemistryBeside:
-            // Beside the transport pass and the mixture collide: more than half a
-            // CU's LDS per block keeps one block, a wavefront per SIMD, on each CU
-            // and leaves the rest of its registers to the other stream, whose
-            // kernels wait on loads.  Unlimited, the chemistry takes every
-            // register first and the two run one after the other: a step of
-            // 131x97x75 cells FP32 1.651 -> 1.597 ms, 128x96x48 FP64 1.960 ->
-            // 1.930 (two blocks: 1.650, 1.946).
-            hipLaunchKernelGGL(k_mc_chemistry<P>, grid1(v.d.n), dim3(BLOCK), 96 * 1024, s, v);
+            hipLaunchKernelGGL(k_mc_chemistry<P>, grid1(v.d.n), dim3(BLOCK), chemistry_alone(v) ? 96 * 1024 : 0, s, v);
             break;
         case McKernel::SpeciesTransport:
             hipLaunchKernelGGL(k_mc_species_transport<P>, dim3(xcd_grid(v.d.n, BLOCK)), dim3(BLOCK), 0, s, v);
@@ -2723,13 +2740,6 @@ void launch_mc_tms_wall(const MultiView<P>& v, const int* cells, int count, hipS
     } else {
         if (count > 0) hipLaunchKernelGGL(k_mc_tms_wall<P>, dim3((count + 63) / 64), dim3(64), 0, s, v, cells, count);
     }
-}
-
-static int cu_count()
-{
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    return cus;
 }
 
 __global__ void k_zero_u32(unsigned* p) { *p = 0u; }
