@@ -1,9 +1,10 @@
 """Large downloads (through the pinned staging) against small ones of the same values.
 
 A grid whose field planes pass the staging threshold is filled with a value
-per cell and read back whole: every field (binary64), species planes and
-populations (binary32 storage with its per-plane shifts), a length that is
-no multiple of the chunk, twice over and from two threads with a context each."""
+per cell and read back whole: fields (binary64), populations (binary32 storage
+with its per-plane shifts), species planes (binary64, and binary32 without a
+shift below and above the threshold), lengths that are no multiple of the chunk,
+twice over and from two threads with a context each."""
 import threading
 import time
 
@@ -20,7 +21,7 @@ def _values(shape, seed):
     return np.random.default_rng(seed).random(shape)
 
 
-@pytest.mark.parametrize("shape", [(126, 127, 131), (127, 130, 125)])  # 17.1 and 16.9 MB planes, odd lengths
+@pytest.mark.parametrize("shape", [(126, 127, 131), (127, 130, 125)])  # 17.57 and 17.30 MB planes, odd lengths
 def test_fields_come_back(shape):
     lat = Lattice(*shape, 0.1, mode=LBM_MODE_STRICT)
     for rep in range(2):
@@ -52,6 +53,16 @@ def test_species_planes_and_populations_come_back(precision):
         else:
             # value - shift in binary32: half a unit in the last place of |f| + |shift| <= 1
             assert np.max(np.abs(a - f)) <= 2.0 ** -24
+    lat.close()
+
+
+def test_binary32_species_planes_come_back():
+    n = (100, 91, 90)  # nine planes of 102 x 93 x 92 binary32 values: 31.4 MB
+    lat = MixtureLattice(*n, *cases.UNITS_FLAME, precision=LBM_FP32_SHIFTED, mode=LBM_MODE_STRICT)
+    for k, name in enumerate(("X", "u")):
+        a = _values((9,) + lat.shape, 8 + k).astype(np.float32).astype(np.float64)
+        lat.set_species_field(name, a)
+        assert np.array_equal(lat.get_species_field(name), a)
     lat.close()
 
 

@@ -129,11 +129,11 @@ def test_fused_reads_between_collide_species_and_streaming():
 
 
 @pytest.mark.parametrize("precision,mode", [(LBM_FP64, LBM_MODE_FUSED), (LBM_FP32_SHIFTED, LBM_MODE_FUSED),
-                                            (LBM_FP32_SHIFTED, LBM_MODE_INPLACE)])
+                                            (LBM_FP32_SHIFTED, LBM_MODE_INPLACE),
+                                            (LBM_FP64, LBM_MODE_STRICT), (LBM_FP32_SHIFTED, LBM_MODE_STRICT)])
 def test_overlapped_step_with_surrogate_matches_serial_calls(precision, mode, monkeypatch):
-    """lbm_step in the fused and in-place modes runs the chemistry (network
-    pass, fallback list) on a second stream beside the transport pass and the
-    mixture collide.  With the same network, envelope and audits, four steps
+    """lbm_step runs the chemistry (network pass, fallback list) on a second
+    stream beside the transport pass and the mixture collide, in every mode.  With the same network, envelope and audits, four steps
     of it are bitwise those of the five calls issued one by one (a context
     created with LBM_AMD_OVERLAP=0 steps serially), surrogate counters
     included."""
