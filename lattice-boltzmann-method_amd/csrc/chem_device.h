@@ -33,9 +33,7 @@ constexpr InvW make_inv_w()
 constexpr InvW INV_W_TABLE = make_inv_w();
 __host__ __device__ inline double inv_w(int a) { return INV_W_TABLE.v[a]; }
 
-// Reciprocal in arithmetic type R: exact for double; for float (the FP32
-// path's binary32 transport) the hardware reciprocal, within 1 ulp.
-__host__ __device__ inline double rcp_r(double x) { return 1.0 / x; }
+// Reciprocal of the FP32 path's binary32 transport: the hardware's, within 1 ulp.
 __host__ __device__ inline float rcp_r(float x)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -553,17 +551,7 @@ __host__ __device__ inline R poly4r(const double c[5], R x)
 {
     return (R)c[0] + x * ((R)c[1] + x * ((R)c[2] + x * ((R)c[3] + x * (R)c[4])));
 }
-template <typename R>
-__host__ __device__ inline R species_viscosity_r(int k, R lnT)
-{
-    return exp(poly4r<R>(VISC_FIT[k], lnT));
-}
-template <typename R>
-__host__ __device__ inline R binary_diff_r(int a, int b, R lnT, R p)
-{
-    if constexpr (sizeof(R) == 4) return exp(poly4r<R>(DIFF_FIT[a][b], lnT)) * rcp_r(p);
-    return quot(exp(poly4r<R>(DIFF_FIT[a][b], lnT)), p);
-}
+__host__ __device__ inline float species_viscosity_f(int k, float lnT) { return exp(poly4r<float>(VISC_FIT[k], lnT)); }
 
 // Divisor sqrt(8 (1 + W_a / W_b)) of the Wilke weights
 __host__ __device__ inline Divisor wilke_divisor(int a, int b)
@@ -609,7 +597,7 @@ __host__ __device__ inline R mix_viscosity_r(R lnT, const double X[NS])
         float mu[NS], sm[NS], rsm[NS];
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
-            mu[k] = species_viscosity_r<float>(k, lnT);
+            mu[k] = species_viscosity_f(k, lnT);
             sm[k] = sqrt(mu[k]);
             rsm[k] = rcp_r(sm[k]);
         }

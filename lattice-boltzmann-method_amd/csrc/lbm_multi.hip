@@ -691,7 +691,7 @@ __device__ __forceinline__ void species_transport_fp32(const MultiView<P>& v, in
     float mu[NS], sm[NS], rsm[NS], den[NS];
 #pragma unroll
     for (int a = 0; a < NS; ++a) {
-        mu[a] = species_viscosity_r<float>(a, lnT);
+        mu[a] = species_viscosity_f(a, lnT);
         sm[a] = sqrtf(mu[a]);
         rsm[a] = rcp_r(sm[a]);
         den[a] = 0.0f;

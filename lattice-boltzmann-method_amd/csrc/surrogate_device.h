@@ -47,7 +47,6 @@ __device__ __forceinline__ uint16_t f2bf(float x)
     __builtin_memcpy(&u, &h, 2);
     return u;
 }
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 // GELU in its tanh form, x (1 + tanh(v)) / 2 with v = sqrt(2/pi) (x + 0.044715
 // x^3), written as x / (1 + exp(-2 v)); and its derivative s + x s (1 - s) 2 v'
