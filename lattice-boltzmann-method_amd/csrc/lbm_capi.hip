@@ -1884,14 +1884,24 @@ namespace {
 // touches; so each kernel sees exactly the inputs of the serial calls and the
 // state is bitwise that of lbm_collide_species followed by lbm_collide and the
 // stream.  Small grids gain most, whose kernels are chains of dependent
-// operations on a few wavefronts.  A step with the chemistry alone beside the
-// rest, and as here: 16x12x10 with two charges 95.5 and 89.7 us, the 2048x4x4
-// flame 505 and 477, the 128x96x48 layer 1925 and 1874.
-// With a network the energy part stays on the step's stream: the network pass
-// is short, and a third kernel beside it stretches it until the chemistry
-// stage takes longer than the integrator's (128x96x64 in FP64: 0.97 of its
-// speed, 1.3 with two streams), for 1 % of the step (256x128x128 in FP32:
-// 6700 us with two streams, 6640 with three).
+// operations on a few wavefronts.
+// A stream of its own costs 7 to 20 us a step in events, so a stream is used only
+// for what is there and gains:
+// * without reaction there is no chemistry stream;
+// * with a network the energy part stays on the step's stream: the network pass
+//   is short, and a third kernel beside it stretches it until the chemistry stage
+//   takes longer than the integrator's (128x96x64 in FP64: 0.97 of its speed, 1.3
+//   with two streams), for 1 % of the step (256x128x128 in FP32: 6700 us with two
+//   streams, 6640 with three);
+// * on binary32 storage, where the mixture collide only starts after the transport
+//   pass, the energy part has a stream of its own above ENERGY_BESIDE_CELLS.  Steps
+//   with it and without, in us, 9 and 6 species, fused: 64^3 inert 384 and 423, 268
+//   and 293, reacting 432 and 471, 285 and 322; 48^3 inert 171 and 174, 122 and 121,
+//   reacting 190 and 189, 132 and 135; 32^3 inert 103 and 91, 83 and 71, reacting 105
+//   and 104, 86 and 82; 6x17x9 inert 82 and 64, 67 and 51, reacting 86 and 74, 76
+//   and 60.  In FP64 it gains from a few thousand cells on (16^3 reacting 101 and
+//   106, 76 and 76; 64^3 777 and 817, 508 and 538).
+constexpr int64_t ENERGY_BESIDE_CELLS = (int64_t)1 << 17;
 int collide_overlapped(lbm_ctx* c)
 {
     HIP_TRY(c, hipSetDevice(c->cfg.device));
@@ -1907,10 +1917,17 @@ int collide_overlapped(lbm_ctx* c)
                     "follow lbm_collide_species");
     const bool chem = c->cfg.reaction;
     const bool push = fused(c) && c->push_ready;
-    HIP_TRY(c, hipEventRecord(c->ev_cstart, c->stream));
-    HIP_TRY(c, hipStreamWaitEvent(c->cstream, c->ev_cstart, 0));
-    const hipStream_t es = c->sur_on ? c->stream : c->estream;
-    if (es != c->stream) HIP_TRY(c, hipStreamWaitEvent(es, c->ev_cstart, 0));
+    const hipStream_t cs = chem ? c->cstream : c->stream;
+    const hipStream_t es =
+        !c->sur_on && (!fp32(c) || c->d.n > ENERGY_BESIDE_CELLS) ? c->estream : c->stream;
+    // what a stream of its own has to wait for: on the FP32 path the mixture
+    // collide takes the transport pass's rates, and follows that pass
+    const bool energy_after_transport = es != c->stream && fp32(c);
+    if (cs != c->stream || (es != c->stream && !energy_after_transport)) {
+        HIP_TRY(c, hipEventRecord(c->ev_cstart, c->stream));
+        if (cs != c->stream) HIP_TRY(c, hipStreamWaitEvent(cs, c->ev_cstart, 0));
+        if (es != c->stream && !energy_after_transport) HIP_TRY(c, hipStreamWaitEvent(es, c->ev_cstart, 0));
+    }
     // the in-place mode's save pass (it reads the species populations and
     // densities, which the other passes leave alone)
     int rc = inplace(c) ? aa_save(c) : LBM_OK;
@@ -1918,28 +1935,27 @@ int collide_overlapped(lbm_ctx* c)
         rc = DISPATCH(c, [&] {
             const MultiView<P> v = make_mview<P>(c, 0, 1);
             if (!c->sur_on)
-                return launch_on(c, c->cstream, "mc_chemistry_plain",
-                                 [&] { launch_mc<P>(McKernel::ChemistryBeside, v, c->cstream); });
-            int r = launch_on(c, c->cstream, "mc_chemistry_surrogate", [&] {
-                launch_mc_sur_chemistry<P>(v, c->net, c->chem_list, c->chem_count, c->cstream);
-            });
+                return launch_on(c, cs, "mc_chemistry_plain",
+                                 [&] { launch_mc<P>(McKernel::ChemistryBeside, v, cs); });
+            int r = launch_on(c, cs, "mc_chemistry_surrogate",
+                              [&] { launch_mc_sur_chemistry<P>(v, c->net, c->chem_list, c->chem_count, cs); });
             if (!r)
-                r = launch_on(c, c->cstream, "mc_chemistry_fallback",
-                              [&] { launch_mc_chem_list<P>(v, c->chem_list, c->chem_count, c->cstream); });
+                r = launch_on(c, cs, "mc_chemistry_fallback",
+                              [&] { launch_mc_chem_list<P>(v, c->chem_list, c->chem_count, cs); });
             return r;
         }());
     // (the joins are recorded whatever happened, so that the step's waits end)
-    const hipError_t ec = hipEventRecord(c->ev_cdone, c->cstream);
+    const hipError_t ec = cs != c->stream ? hipEventRecord(c->ev_cdone, cs) : hipSuccess;
     if (!rc) rc = run_mc(c, McKernel::SpeciesTransport, "mc_species_transport", 0, 1);
     c->omix_fresh = !rc && fp32(c);
     hipError_t ee = hipSuccess;
-    if (c->omix_fresh && es != c->stream) {
+    if (energy_after_transport) {
         ee = hipEventRecord(c->ev_trans, c->stream);
         if (ee == hipSuccess) ee = hipStreamWaitEvent(es, c->ev_trans, 0);
     }
-    if (!rc) rc = run_mc_on(c, es, McKernel::Collide, "mc_collide_mixture", 0, 1);
+    if (!rc && ee == hipSuccess) rc = run_mc_on(c, es, McKernel::Collide, "mc_collide_mixture", 0, 1);
     HIP_TRY(c, ec);
-    HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_cdone, 0));
+    if (cs != c->stream) HIP_TRY(c, hipStreamWaitEvent(c->stream, c->ev_cdone, 0));
     if (!rc && inplace(c)) {
         rc = aa_collide_species(c);
     } else if (!rc && push) {
@@ -1950,7 +1966,7 @@ int collide_overlapped(lbm_ctx* c)
     }
     // (queued last: a step whose species collide is refused, for instance for
     // want of memory, leaves the energy populations where lbm_collide does)
-    const bool energy = !rc && (push || inplace(c));
+    const bool energy = !rc && ee == hipSuccess && (push || inplace(c));
     if (energy) rc = run_mc_on(c, es, McKernel::StreamEnergy, "mc_stream_energy", 1, 0);
     if (ee == hipSuccess && es != c->stream) ee = hipEventRecord(c->ev_edone, es);
     HIP_TRY(c, ee);
