@@ -390,7 +390,10 @@ __device__ inline void capture_row(const MultiView<P>& v, const ChemState& s, co
 }
 
 // waves per SIMD the plain chemistry is built for (a large mechanism's
-// per-cell arrays would spill)
+// per-cell arrays would spill).  One build serves all grids: where there are fewer
+// wavefronts than SIMDs a single wave's registers gain little (a step of the
+// 2048x4x4 flame 315 us with three waves and 313 with one, of 16x12x10 cells 90
+// and 90), and 128x96x48 cells lose (1.840 ms and 1.905).
 constexpr int CHEM_WAVES = NS <= 16 ? 3 : 1;
 
 // Plain chemistry of every fluid cell; optionally samples (state, result)
@@ -1117,7 +1120,10 @@ __global__ __launch_bounds__(BLOCK) void k_mc_side_push_aa(MultiView<P> v)
 enum : int { OMIX_OM = 0, OMIX_OM1 = 1, OMIX_THETA = 2, OMIX_USHIFT = 3, OMIX_DQ = 4, OMIX_PLANES = 7 };
 
 // The FP64 form holds 174 VGPRs by itself; three waves (168, 28 B of scratch)
-// took 284 us against 317 with two on 128x96x48 cells.
+// took 284 us against 317 with two on 128x96x48 cells.  Steps with three waves, and
+// without the limit and its species loops unrolled: 128x96x48 1.840 and 1.866 ms, and
+// where there are fewer wavefronts than SIMDs 2048x4x4 flame 315 and 312 us,
+// 16x12x10 90 and 87; one build serves both.
 template <typename P, int PART>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(P) == 8 && PART == 0 && NS <= 16 ? 3 : 1, 8)))
 void k_mc_collide(MultiView<P> v)
